@@ -93,6 +93,42 @@ def test_ties_zero_rows_fp16_and_strides():
     assert_same_as_oracle(t, q, s)
 
 
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize('k', [1, 3, 7, 8, 65, 511, 513, 1030, 2049, 4095, 4097, 9001, 16383, 16385, 33000])
+def test_row_lengths(dtype, k):
+    """Row lengths at the edges of every form (shorter than a 16-byte chunk, each register count, one wavefront or a
+    block per row, rows read twice), rows off 16-byte alignment, and the rows the multiplying form leaves to the
+    division or must not change: infinities, NaN, zeros, the largest and the smallest steps, and a step whose
+    significand is all ones."""
+    from efficientgpt_amd.int8_linear import quantize_weight
+    g = torch.Generator().manual_seed(k)
+    w = torch.randn(13, k + 1, generator=g) * torch.logspace(-3, 3, 13)[:, None]
+    w = w.to(dtype)[:, 1:]
+    w[3] = 0
+    if dtype is torch.float32:
+        w[4] *= 1e33
+        w[5] *= 1e-12
+        # 127 (2 - 2^-23) rounds to a multiple whose 127th is 2 - 2^-23 again: a step of 24 ones
+        w[6, 0] = 127 * (2 - 2.0 ** -23)
+        w[6, 1:] = w[6, 1:].clamp(-200, 200)
+    w = w.contiguous() if k % 2 else w
+    finite = torch.cat([w, w])[:13].cuda()
+    q, s = quantize_weight(finite)
+    assert_same_as_oracle(finite, q, s)
+    w[1, k // 2] = float('inf')
+    w[2, k - 1] = float('nan')
+    d = w.cuda()
+    q, s = quantize_weight(d)
+    keep = [r for r in range(13) if r not in (1, 2)]
+    assert_same_as_oracle(d[keep], q[keep], s[keep])
+    # an infinite step makes every finite value's quotient 0 and the infinity's NaN; a NaN step makes all NaN; the
+    # kernel's clamp takes NaN to -127
+    assert float(s[1]) == float('inf') and bool(torch.isnan(s[2]))
+    want = torch.zeros(k, dtype=torch.int8)
+    want[k // 2] = -127
+    assert torch.equal(q[1].cpu(), want) and bool((q[2] == -127).all())
+
+
 def test_quantize_model_on_gpu_matches_oracle_codes():
     transformers = pytest.importorskip('transformers')
     from efficientgpt_amd.int8_linear import Int8Linear, quantize_model
