@@ -118,6 +118,10 @@ __device__ __forceinline__ uint32_t lds_addr(const void* p) {
 __device__ __forceinline__ void lds_load16(uint32_t lds_base, const void* g) {
   asm volatile("global_load_lds_dwordx4 %0, off" : : "v"(g), "{m0}"(lds_base) : "memory");
 }
+// The same from a wave-uniform base and a 32-bit byte offset per lane.
+__device__ __forceinline__ void lds_load16_at(uint32_t lds_base, const void* base, uint32_t off) {
+  asm volatile("global_load_lds_dwordx4 %0, %1" : : "v"(off), "s"(base), "{m0}"(lds_base) : "memory");
+}
 __device__ __forceinline__ void lds_load4(uint32_t lds_base, const void* g) {
   asm volatile("global_load_lds_dword %0, off" : : "v"(g), "{m0}"(lds_base) : "memory");
 }

@@ -6,22 +6,15 @@
 // GEMM of x with the exact bf16 image of the int8 weights (fp32 accumulation,
 // rounded once to bf16), then the per-row scale in fp32 and a second bf16
 // rounding. The reference materialises w.to(bfloat16) and calls the library
-// GEMM; here the int8 rows go through LDS as int8 and each wavefront converts
-// its fragments to bf16 in registers, so the weights cross HBM once, as int8.
+// GEMM; here the weights are converted on the chip, so they cross HBM once, as int8.
 //
 // Design:
-//   * A block of 4 or 8 wavefronts computes a BM x BN tile of y; each wavefront
-//     owns a grid of 32 x 32 tiles of v_mfma_f32_32x32x16_bf16 (fp32
-//     accumulators, bf16 products exact).
-//   * K advances 64 (128 in the split slices) at a time through two LDS buffers
-//     and two register staging sets: the global loads of step k + 2 are issued
-//     before the MFMAs of step k; one barrier per step.
-//   * x rows sit in LDS as bf16 (BK + 8 padding). Weights are converted to bf16
-//     once per block by the thread that loaded them, as it writes them to LDS (the
-//     tiles with two wavefronts along M, which read the same fragments), or stay
-//     int8 (BK + 16 padding) and each wavefront converts the 8-byte fragments it
-//     reads (the 128 x 256 tile, whose wavefronts lie along N). The padding puts
-//     the fragment reads of 16 consecutive rows on distinct banks.
+//   * Large products run tiles of 128 x 128 to 256 x 256 on v_mfma_f32_16x16x32_bf16 (int8_gemm_dma_kernel): operands
+//     straight into LDS, the weights as int8, eight wavefronts whose two halves take turns at the matrix cores.
+//   * Small ones run 64 x 64 and 128 x 64 tiles of 4 wavefronts on v_mfma_f32_32x32x16_bf16 (int8_gemm_kernel). K
+//     advances 64 (128 where the tiles are few) at a time through two LDS buffers and two register staging sets: the
+//     global loads of step k + 2 are issued before the MFMAs of step k; one barrier per step. The padding of the LDS
+//     rows puts the fragment reads of 16 consecutive rows on distinct banks.
 //   * int8 -> bf16 is exact: every value in [-127, 127] is a bf16.
 //   * Rows past M or N read a valid row and are never stored.
 //   * Split-K (short M, long K: too few output tiles to give every CU a block):
@@ -29,10 +22,11 @@
 //     workspace [splits][M][N]; a second kernel adds the slices in split order and
 //     applies the two roundings. The fp32 sum is the same product in another
 //     order, as any GEMM blocking is.
-// Operand layouts (checked on the MI355X): lane l holds A[l % 32][8 (l / 32) + e]
+// Operand layouts of v_mfma_f32_32x32x16_bf16 (checked on the MI355X): lane l holds A[l % 32][8 (l / 32) + e]
 // and B[8 (l / 32) + e][l % 32], e = 0..7; accumulator register r of lane l is
 // C[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
 #include <algorithm>
+#include <type_traits>
 
 #include "common.h"
 
@@ -41,6 +35,8 @@ namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float f32x16 __attribute__((ext_vector_type(16)));
+typedef float f32x4 __attribute__((ext_vector_type(4)));
+typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
 constexpr int kBK = 64;        // K per LDS stage of the one-pass kernel: K must be a multiple of it
 constexpr int kBKSplit = 128;  // K per LDS stage of the split-K slices (half the dependent steps)
@@ -51,8 +47,7 @@ struct GemmShape {
   static constexpr int WM = NW / WN;          // wavefronts along M (the block's NW as WM x WN)
   static constexpr int TM = BM / (32 * WM);  // 32 x 32 tiles per wavefront along M
   static constexpr int TN = BN / (32 * WN);  // ... along N
-  static constexpr int kLdsRow = BK + 8;    // bf16 elements per x row in LDS (16 bytes of padding)
-  static constexpr int kLdsRowW = BK + 16;  // bytes per int8 weight row in LDS (16 bytes of padding)
+  static constexpr int kLdsRow = BK + 8;    // bf16 elements per x or weight row in LDS (16 bytes of padding)
   static constexpr int kALoads = BM * BK * 2 / (NT * 16);  // 16-byte x loads per thread per step
   static constexpr int kBLoads = BN * BK / (NT * 16);      // 16-byte int8 loads per thread per step
   static_assert(WM * WN == NW && TM >= 1 && TN >= 1 && kALoads >= 1 && kBLoads >= 1, "tile too small for the block");
@@ -90,9 +85,8 @@ struct GemmArgs {
   int inter;           // SwiGLU form: features (w holds inter gate rows, then inter up rows; N = 2 inter)
 };
 
-// SwiGLU form: block tile column j (of BN) -> weight row. Each wavefront's BN / WN columns hold half of its
-// features' gate rows and then the same features' up rows, so gate and up of a feature land in the same lane
-// and accumulator register of a wavefront's tiles tn and tn + TN / 2. Features past `inter` read the last one.
+// SwiGLU form of the small tiles: block tile column j (of BN) -> weight row. Each wavefront's BN / WN columns hold its
+// features' gate rows and then the same features' up rows. Features past `inter` read the last one.
 template <int BN, int WN>
 __device__ __forceinline__ int64_t swiglu_row(int64_t pid_n, int j, int inter) {
   constexpr int kPerWave = BN / WN, kHalf = kPerWave / 2;
@@ -100,17 +94,6 @@ __device__ __forceinline__ int64_t swiglu_row(int64_t pid_n, int j, int inter) {
   const int64_t f = min(pid_n * (BN / 2) + wn * kHalf + (o % kHalf), (int64_t)inter - 1);
   return o < kHalf ? f : inter + f;
 }
-
-// Wavefronts of the 128 x 256 and 128 x 128 tiles, and how many of them lie along N.
-constexpr int kNW256 = 4;
-constexpr int kWN256 = 4;
-constexpr int kNW128 = 8;
-constexpr int kWN128 = 4;
-
-// Blocks per CU the register allocation must allow (launch bounds): two for the
-// 128 x 256 tile.
-template <int BM, int BN, int NW>
-constexpr int kGemmMinBlocks = (BM == 128 && BN == 256 && NW == 4) ? 2 : 1;
 
 constexpr int kXcds = 8;        // MI355X: 8 XCDs, each with its own L2
 constexpr int kGroupM = 8;      // M tiles per group of the tile order
@@ -171,31 +154,6 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& a, const f32x16 (&acc
       }
     }
     return;
-  } else if constexpr (SWIGLU) {
-    // act = bf16(bf16(silu(g)) * u) with g and u the product's two roundings (the reference's prefill formula
-    // for each), SwiGLU rounded as transformers' bf16 Qwen3MLP (models/qwen3/modeling_qwen3.py:49-62): the same
-    // arithmetic per element as the GEMM followed by egpt_silu_mul.
-#pragma unroll
-    for (int tn = 0; tn < TN / 2; ++tn) {
-      const int64_t f = (int64_t)pid_n * (BN / 2) + (wave % WN) * (BN / WN / 2) + tn * 32 + lane % 32;
-      const int64_t fc = min(f, (int64_t)a.inter - 1);
-      const float sg_scale = a.scale[fc], su_scale = a.scale[a.inter + fc];
-      const uint32_t base = (uint32_t)((mrow0 * a.ldy + f) * 2);
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) {
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int dm = tm * 32 + 8 * (r / 4) + r % 4;
-          if (mrow0 + dm < a.M && f < a.inter) {
-            const float g = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][tn][r])) * sg_scale));
-            const float u = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][tn + TN / 2][r])) * su_scale));
-            const float sg = bf16_to_f32(f32_to_bf16(g / (1.0f + expf(-g))));
-            *(uint16_t*)(yb + (base + (uint32_t)dm * pitch)) = f32_to_bf16(sg * u);
-          }
-        }
-      }
-    }
-    return;
   }
 #pragma unroll
   for (int tn = 0; tn < TN; ++tn) {
@@ -216,24 +174,16 @@ __device__ __forceinline__ void gemm_store(const GemmArgs& a, const f32x16 (&acc
   }
 }
 
-// BF16B: the weights are converted to bf16 once, by the thread that loaded them,
-// as they are written to LDS, and the wavefronts read bf16 fragments; otherwise
-// they stay int8 in LDS and every wavefront converts the fragments it reads (the
-// wavefronts along M convert the same fragment each). BF16B doubles the weights'
-// LDS space and read bytes.
-template <int BM, int BN, int BK, bool SPLIT, int WN, int NW, bool SWIGLU = false, bool BF16B = false>
-__global__ __launch_bounds__(NW * kWave, (kGemmMinBlocks<BM, BN, NW>)) void int8_gemm_kernel(const GemmArgs a) {
+// The small tiles (64 x 64 and 128 x 64): the weights are converted to bf16 once, by the thread that loaded them, as
+// they are written to LDS, and the wavefronts read bf16 fragments.
+template <int BM, int BN, int BK, bool SPLIT, int WN, int NW, bool SWIGLU = false>
+__global__ __launch_bounds__(NW * kWave, 1) void int8_gemm_kernel(const GemmArgs a) {
   using S = GemmShape<BM, BN, BK, WN, NW>;
   constexpr int TM = S::TM, TN = S::TN;
-  static_assert(!SWIGLU || (!SPLIT && (TN % 2 == 0 || TN == 1)),
-                "the SwiGLU form pairs a wavefront's column tiles, or the two halves of its one tile");
-  constexpr int kLdsRow = S::kLdsRow, kLdsRowW = S::kLdsRowW;
-  // weight row pitch in LDS: bytes (int8) or bf16 elements (BF16B, the x rows' pitch)
-  constexpr int kBRow = BF16B ? kLdsRow : kLdsRowW;
+  static_assert(!SWIGLU || (!SPLIT && TN == 1), "the SwiGLU form pairs the two halves of a wavefront's one column tile");
+  constexpr int kLdsRow = S::kLdsRow;
   __shared__ __align__(16) uint16_t As[2][BM * kLdsRow];
-  __shared__ __align__(16) char Bsm[2][BF16B ? BN * kLdsRow * 2 : BN * kLdsRowW];
-  int8_t(&Bs)[2][BN * kLdsRowW] = *reinterpret_cast<int8_t(*)[2][BN * kLdsRowW]>(&Bsm);
-  uint16_t(&Bs16)[2][BN * kLdsRow] = *reinterpret_cast<uint16_t(*)[2][BN * kLdsRow]>(&Bsm);
+  __shared__ __align__(16) uint16_t Bs[2][BN * kLdsRow];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
@@ -269,7 +219,7 @@ __global__ __launch_bounds__(NW * kWave, (kGemmMinBlocks<BM, BN, NW>)) void int8
     const int row = i / (BK / 16), chunk = i % (BK / 16);
     const int64_t wrow = SWIGLU ? swiglu_row<BN, WN>(pid_n, row, a.inter) : min(n0 + row, (int64_t)a.N - 1);
     woff[j] = (uint32_t)(wrow * a.ldw + kbeg + chunk * 16);
-    b_lds[j] = row * kBRow + chunk * 16;
+    b_lds[j] = row * kLdsRow + chunk * 16;
   }
   // Two register staging sets: the loads of step k + 2 are issued while step k is
   // multiplied and land in LDS among the MFMAs of step k + 1, one to two steps of
@@ -284,23 +234,15 @@ __global__ __launch_bounds__(NW * kWave, (kGemmMinBlocks<BM, BN, NW>)) void int8
 #pragma unroll
     for (int j = 0; j < S::kBLoads; ++j) wr[set][j] = ld16_stream(wb + (woff[j] + k0));
   };
-  // Part q of Q of the LDS stores of one K step (the staging loads j with j % Q == q).
-  auto store_part = [&](int buf, int set, int q, int Q) {
+  auto store_step = [&](int buf, int set) {
 #pragma unroll
-    for (int j = 0; j < S::kALoads; ++j)
-      if (j % Q == q) *(u32x4*)&As[buf][a_lds[j]] = xr[set][j];
+    for (int j = 0; j < S::kALoads; ++j) *(u32x4*)&As[buf][a_lds[j]] = xr[set][j];
 #pragma unroll
     for (int j = 0; j < S::kBLoads; ++j) {
-      if (j % Q != q) continue;
-      if constexpr (BF16B) {
-        *(bf16x8*)&Bs16[buf][b_lds[j]] = int8x8_to_bf16(wr[set][j].x, wr[set][j].y);
-        *(bf16x8*)&Bs16[buf][b_lds[j] + 8] = int8x8_to_bf16(wr[set][j].z, wr[set][j].w);
-      } else {
-        *(u32x4*)&Bs[buf][b_lds[j]] = wr[set][j];
-      }
+      *(bf16x8*)&Bs[buf][b_lds[j]] = int8x8_to_bf16(wr[set][j].x, wr[set][j].y);
+      *(bf16x8*)&Bs[buf][b_lds[j] + 8] = int8x8_to_bf16(wr[set][j].z, wr[set][j].w);
     }
   };
-  auto store_step = [&](int buf, int set) { store_part(buf, set, 0, 1); };
 
   f32x16 acc[TM][TN];
 #pragma unroll
@@ -314,73 +256,28 @@ __global__ __launch_bounds__(NW * kWave, (kGemmMinBlocks<BM, BN, NW>)) void int8
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm) a_frag[tm] = (wm0 + tm * 32 + lane % 32) * kLdsRow + frag_k;
 #pragma unroll
-  for (int tn = 0; tn < TN; ++tn) b_frag[tn] = (wn0 + tn * 32 + lane % 32) * kBRow + frag_k;
+  for (int tn = 0; tn < TN; ++tn) b_frag[tn] = (wn0 + tn * 32 + lane % 32) * kLdsRow + frag_k;
 
-  // The MFMAs of one K step from LDS buffer `buf`, 16 K columns at a time. With
-  // sbuf >= 0 (large tiles) the next step's LDS stores (staging set `set` into
-  // buffer sbuf) are spread over the K sub-steps, after each one's MFMAs, so their
-  // conversions and writes run while the MFMAs do instead of after them.
+  // The MFMAs of one K step from LDS buffer `buf`, then, with sbuf >= 0, the next step's LDS stores (staging set `set`
+  // into buffer sbuf). One wavefront per SIMD with a short MFMA chain per 16 columns leaves nothing to cover an LDS
+  // read issued just before its MFMA, so every fragment of the step is read first.
   auto mma_step = [&](int buf, int sbuf = -1, int set = 0) {
-    if constexpr (TM * TN <= 2) {
-      // Small tiles run one wavefront per SIMD with a short MFMA chain per K sub-step, so
-      // nothing would cover an LDS read issued just before its MFMA: read every fragment
-      // of the step first, then convert and multiply.
-      bf16x8 af[BK / 16][TM];
-      uint32_t bw[BK / 16][TN][2];
-      bf16x8 bh[BK / 16][TN];
+    bf16x8 af[BK / 16][TM], bh[BK / 16][TN];
 #pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
+    for (int ks = 0; ks < BK / 16; ++ks) {
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) af[ks][tm] = *(const bf16x8*)&As[buf][a_frag[tm] + ks * 16];
+      for (int tm = 0; tm < TM; ++tm) af[ks][tm] = *(const bf16x8*)&As[buf][a_frag[tm] + ks * 16];
 #pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-          if constexpr (BF16B) {
-            bh[ks][tn] = *(const bf16x8*)&Bs16[buf][b_frag[tn] + ks * 16];
-          } else {
-            const uint32_t* p = (const uint32_t*)&Bs[buf][b_frag[tn] + ks * 16];
-            bw[ks][tn][0] = p[0];
-            bw[ks][tn][1] = p[1];
-          }
-        }
-      }
+      for (int tn = 0; tn < TN; ++tn) bh[ks][tn] = *(const bf16x8*)&Bs[buf][b_frag[tn] + ks * 16];
+    }
 #pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
-        bf16x8 bfr[TN];
+    for (int ks = 0; ks < BK / 16; ++ks)
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
-          bfr[tn] = BF16B ? bh[ks][tn] : int8x8_to_bf16(bw[ks][tn][0], bw[ks][tn][1]);
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks][tm], bfr[tn], acc[tm][tn], 0, 0, 0);
-      }
-    } else {
-#pragma unroll
-      for (int ks = 0; ks < BK / 16; ++ks) {
-        bf16x8 af[TM], bfr[TN];
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm) af[tm] = *(const bf16x8*)&As[buf][a_frag[tm] + ks * 16];
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn) {
-          if constexpr (BF16B) {
-            bfr[tn] = *(const bf16x8*)&Bs16[buf][b_frag[tn] + ks * 16];
-          } else {
-            const uint32_t* p = (const uint32_t*)&Bs[buf][b_frag[tn] + ks * 16];
-            bfr[tn] = int8x8_to_bf16(p[0], p[1]);
-          }
-        }
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[tm], bfr[tn], acc[tm][tn], 0, 0, 0);
-        if (sbuf >= 0) store_part(sbuf, set, ks, BK / 16);
-      }
-    }
-    if constexpr (TM * TN <= 2) {
-      if (sbuf >= 0) store_step(sbuf, set);
-    }
+          acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks][tm], bh[ks][tn], acc[tm][tn], 0, 0, 0);
+    if (sbuf >= 0) store_step(sbuf, set);
   };
 
   load_step(0, 0);
@@ -425,137 +322,239 @@ __global__ __launch_bounds__(NW * kWave, (kGemmMinBlocks<BM, BN, NW>)) void int8
   gemm_store<BM, BN, TM, TN, WN, SWIGLU>(a, acc, m0, n0, wm0, wn0, pid_n, lane, wave);
 }
 
-// The 256 x 256 tile with its operands loaded straight into LDS (global_load_lds_dwordx4), three K steps of 64
-// in flight: the loads of step k + 2 are issued as step k starts, with no staging registers and no LDS stores by
-// the wavefronts, and each step waits only for its own loads. A step's stage holds the x rows as bf16 (128
-// bytes a row) and the weight rows as int8 (64 bytes a row), 48 KiB; every wavefront converts the weight
-// fragments it reads. Rows carry no padding: the 16-byte chunks of x row r sit at chunk c ^ dma_aswz(r) and those
-// of weight row n at c ^ dma_bswz(n), so the 16 lanes that a 16-byte LDS read serves together ({0-3, 12-15,
-// 20-23, 24-27} or {4-7, 8-11, 16-19, 28-31} of a half wavefront, measured on the MI355X) fall on distinct banks.
-// Each 16-byte weight read feeds two MFMAs: the MFMA k index 8 h + e of sub-step u of K pair p stands for the
-// step's column 32 p + 16 h + 8 u + e in both operands (a permutation of the sum's terms within the step).
+// The large tiles: 32 TM x 64 TN of y per block, eight wavefronts as 2 (M) x 4 (N) of 16 TM x 16 TN each.
+//
+// v_mfma_f32_16x16x32_bf16, not 32x32x16: over random operands in registers the chip sustains 1.90 PFLOP/s of the
+// former and 1.37 of the latter (on zeros 2.45 and 1.65). The weights are the A operand, so an accumulator's four
+// registers are four consecutive columns of one x row, and the weight rows of a wavefront's tiles are dealt so that
+// lane l ends with the 4 TN consecutive columns from 4 TN (l / 16): each row is stored in 16-byte pieces.
+//
+// Operands go straight into LDS (global_load_lds_dwordx4), x rows as bf16 and weight rows as int8, through three
+// stages of 64 K columns, the loads of step k + 2 issued as step k starts. Each 16-byte weight read feeds two MFMAs:
+// the MFMA k index 8 h + e of half u stands for the step's column 16 h + 8 u + e in both operands.
+//
+// What bounded the kernel was each SIMD's two wavefronts reading LDS, converting and multiplying in the same phase
+// (MFMA busy 51% of the time). Here they take turns: wavefronts 4-7 run one barrier behind 0-3, so that on every SIMD
+// one wavefront reads and converts a whole step's fragments while the other, at raised issue priority, does nothing
+// but the 2 TM TN MFMAs of its own. Conversions moved among the MFMAs instead cost 8% (256 x 256 tile), 32-column
+// phases 1-2%. MFMA busy 68%, at a clock of 1.92 GHz: the chip's power is the next bound.
+// Measured on the MI355X (us, the former 32x32x16 kernel with all wavefronts in one phase -> this): 8192 x 4096 ->
+// 24576 1476-1491 -> 1203 (1.37 PFLOP/s), 8192 x 4096 -> 6144 374 -> 296, 6001 x 12288 -> 4096 608 -> 484, 1000 x
+// 4096 -> 24576 233 -> 175 and -> 6144 72 -> 60, 300 x 2048 -> 12288 36.6 -> 28.3.
 constexpr int kDmaBK = 64;
 constexpr int kDmaWaves = 8;
 constexpr int kDmaStages = 3;
-constexpr int kDmaARow = kDmaBK * 2;                          // bytes per x row of a stage
-constexpr int kDmaBRow = kDmaBK;                              // bytes per weight row of a stage
-constexpr int kDmaAStage = 256 * kDmaARow;                    // 32 KiB
-constexpr int kDmaStage = kDmaAStage + 256 * kDmaBRow;        // 48 KiB
-constexpr int kDmaALoads = kDmaAStage / (kDmaWaves * 1024);   // 1 KiB loads per wavefront and step: 4
-constexpr int kDmaBLoads = 256 * kDmaBRow / (kDmaWaves * 1024);  // 2
 
-__device__ __forceinline__ int dma_aswz(int r) { return (r >> 1) & 7; }
-__device__ __forceinline__ int dma_bswz(int n) { return (n >> 2) & 3; }
+// LDS positions of the 16-byte chunks: chunk c of x row r sits at c ^ dma_aswz(r), chunk c of weight row n (t = the
+// row's group of 4 TN within its wavefront's 16 TN rows) at c ^ dma_bswz(t). A 16-byte LDS read serves 16 lanes
+// together ({0-3, 12-15, 20-23, 24-27} or {4-7, 8-11, 16-19, 28-31} of a half wavefront, measured on the MI355X);
+// with these both operands' fragment reads put them on distinct banks.
+__device__ __forceinline__ int dma_aswz(int r) { return ((r >> 1) & 1) | (((r >> 3) & 1) << 2); }
+__device__ __forceinline__ int dma_bswz(int t) { return ((t & 1) << 1) ^ (3 * ((t >> 1) & 1)); }
 
-template <bool SWIGLU>
+typedef uint32_t u32x4_h __attribute__((ext_vector_type(4), aligned(2)));
+typedef uint32_t u32x2_h __attribute__((ext_vector_type(2), aligned(2)));
+
+// C consecutive outputs of row m from column c0, rounded to bf16: 16- and 8-byte stores at any element alignment, or one
+// by one where the row ends among them.
+template <int C>
+__device__ __forceinline__ void store_row(const GemmArgs& a, int64_t m, int64_t c0, int64_t cols, const float (&o)[C]) {
+  if (m >= a.M) return;
+  uint16_t* p = a.y + m * a.ldy + c0;
+  if (c0 + C <= cols) {
+    uint32_t w[C / 2];
+#pragma unroll
+    for (int i = 0; i < C / 2; ++i) w[i] = pack2_bf16(o[2 * i], o[2 * i + 1]);
+#pragma unroll
+    for (int i = 0; i + 4 <= C / 2; i += 4)
+      *(global_ptr<u32x4_h>)(p + 2 * i) = u32x4{w[i], w[i + 1], w[i + 2], w[i + 3]};
+    if constexpr (C % 8)
+      *(global_ptr<u32x2_h>)(p + C - 4) = u32x2{w[C / 2 - 2], w[C / 2 - 1]};
+  } else {
+#pragma unroll
+    for (int i = 0; i < C; ++i)
+      if (c0 + i < cols) gstore(p + i, f32_to_bf16(o[i]));
+  }
+}
+
+template <int TM, int TN, bool SWIGLU>
 __global__ __launch_bounds__(kDmaWaves * kWave, 1) void int8_gemm_dma_kernel(const GemmArgs a) {
-  constexpr int BM = 256, BN = 256, WN = 4, WM = kDmaWaves / WN;
-  constexpr int TM = BM / (32 * WM), TN = BN / (32 * WN);  // 4 x 2 tiles of 32 x 32 per wavefront
-  __shared__ __align__(16) char smem[kDmaStages * kDmaStage];
+  constexpr int WN = 4, BM = 32 * TM, BN = 64 * TN;
+  constexpr int kARow = kDmaBK * 2, kBRow = kDmaBK;  // bytes per x row / weight row of a stage
+  constexpr int kAStage = BM * kARow, kStage = kAStage + BN * kBRow;
+  constexpr int kALoads = kAStage / (kDmaWaves * 1024);             // 1 KiB loads per wavefront and step
+  constexpr int kBBlocks = BN * kBRow / 1024;                       // 1 KiB weight loads per step, over the block
+  constexpr int kBLoads = (kBBlocks + kDmaWaves - 1) / kDmaWaves;   // per wavefront, the last one maybe not
+  constexpr bool kBEven = kBBlocks % kDmaWaves == 0;
+  static_assert(TM % 2 == 0 && (!SWIGLU || TN % 2 == 0), "");
+  __shared__ __align__(16) char smem[kDmaStages * kStage];
 
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-  const int wm0 = (wave / WN) * (BM / WM);
-  const int wn0 = (wave % WN) * (BN / WN);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm0 = (wave / WN) * (16 * TM);
+  const int wn0 = (wave % WN) * (16 * TN);
   int pid_m, pid_n;
   gemm_tile((int)blockIdx.x, a.tiles_m, a.tiles_n, pid_m, pid_n);
   const int64_t m0 = (int64_t)pid_m * BM;
   const int64_t n0 = (int64_t)pid_n * BN;
 
-  // Load q of a wavefront fills 1 KiB block wave * loads + q of its operand's stage: 8 x rows (lane i: row i / 8,
-  // stored chunk i % 8) or 16 weight rows (lane i: row i / 4, stored chunk i % 4). 32-bit byte offsets from the
-  // operands' bases (the host checks that both span < 2 GiB); rows past M or N read the last one.
-  const char* xb = (const char*)a.x;
-  const char* wb = (const char*)a.w;
-  uint32_t xo[kDmaALoads], wo[kDmaBLoads];
+  // 32-bit byte offsets from the operands' bases (the host checks that both span < 2 GiB); rows past M or N read the
+  // last one.
+  uint32_t xo[kALoads], wo[kBLoads];
 #pragma unroll
-  for (int q = 0; q < kDmaALoads; ++q) {
-    const int row = (wave * kDmaALoads + q) * 8 + lane / 8;
+  for (int q = 0; q < kALoads; ++q) {
+    const int row = (wave * kALoads + q) * 8 + lane / 8;
     const int c = (lane % 8) ^ dma_aswz(row);
     xo[q] = (uint32_t)((min(m0 + row, (int64_t)a.M - 1) * a.ldx + 8 * c) * 2);
   }
+  // Tile column j -> weight row. SwiGLU: each lane's 4 TN columns are 2 TN features' gate rows, then their up rows.
 #pragma unroll
-  for (int q = 0; q < kDmaBLoads; ++q) {
-    const int row = (wave * kDmaBLoads + q) * 16 + lane / 4;
-    const int c = (lane % 4) ^ dma_bswz(row);
-    const int64_t wrow = SWIGLU ? swiglu_row<BN, WN>(pid_n, row, a.inter) : min(n0 + row, (int64_t)a.N - 1);
+  for (int q = 0; q < kBLoads; ++q) {
+    const int row = (q * kDmaWaves + wave) * 16 + lane / 4;
+    const int c = (lane % 4) ^ dma_bswz((row / (4 * TN)) % 4);
+    int64_t wrow;
+    if constexpr (SWIGLU) {
+      const int o = row % (4 * TN);
+      const int64_t f = min((int64_t)pid_n * (BN / 2) + row / (4 * TN) * (2 * TN) + o % (2 * TN), (int64_t)a.inter - 1);
+      wrow = o < 2 * TN ? f : a.inter + f;
+    } else {
+      wrow = min(n0 + row, (int64_t)a.N - 1);
+    }
     wo[q] = (uint32_t)(wrow * a.ldw + 16 * c);
   }
   const uint32_t sbase = lds_addr(smem);
   auto issue = [&](int kt, int stage) {
-    const uint32_t k0 = (uint32_t)(kt * kDmaBK);
-    const uint32_t abase = sbase + (uint32_t)(stage * kDmaStage);
+    const uint32_t abase = sbase + (uint32_t)(stage * kStage);
+    const char* xb = (const char*)a.x + (int64_t)kt * kARow;
+    const char* wb = (const char*)a.w + (int64_t)kt * kBRow;
 #pragma unroll
-    for (int q = 0; q < kDmaALoads; ++q)
-      lds_load16(abase + (uint32_t)((wave * kDmaALoads + q) * 1024), xb + (xo[q] + 2 * k0));
+    for (int q = 0; q < kALoads; ++q) lds_load16_at(abase + (uint32_t)((wave * kALoads + q) * 1024), xb, xo[q]);
 #pragma unroll
-    for (int q = 0; q < kDmaBLoads; ++q)
-      lds_load16(abase + (uint32_t)(kDmaAStage + (wave * kDmaBLoads + q) * 1024), wb + (wo[q] + k0));
+    for (int q = 0; q < kBLoads; ++q)
+      if (kBEven || q * kDmaWaves + wave < kBBlocks)
+        lds_load16_at(abase + (uint32_t)(kAStage + (q * kDmaWaves + wave) * 1024), wb, wo[q]);
   };
+  // Wait until at most the loads of S steps are in flight.
+  auto wait_steps = [&](auto S) {
+    if (kBEven || wave < kBBlocks % kDmaWaves)
+      EGPT_WAIT_VMCNT(decltype(S)::value * (kALoads + kBLoads));
+    else
+      EGPT_WAIT_VMCNT(decltype(S)::value * (kALoads + kBLoads - 1));
+  };
+  using One = std::integral_constant<int, 1>;
 
-  // Fragment reads: the swizzles depend on row bits that the wavefront and tile origins (multiples of 32) leave
-  // alone, so each lane's chunk offsets are fixed.
-  const int r32 = lane % 32, h = lane / 32;
-  const int arow = (wm0 + r32) * kDmaARow;               // + tm * 32 rows
-  const int brow = kDmaAStage + (wn0 + r32) * kDmaBRow;  // + tn * 32 rows
-  int ach[2][2], bch[2];
-#pragma unroll
-  for (int p = 0; p < 2; ++p) {
-    bch[p] = 16 * ((2 * p + h) ^ dma_bswz(r32));
-#pragma unroll
-    for (int u = 0; u < 2; ++u) ach[p][u] = 16 * ((4 * p + 2 * h + u) ^ dma_aswz(r32));
-  }
+  const int r16 = lane % 16, h = lane / 16;
+  // Weight row of tile tn's slot i: 4 TN (i / 4) + 4 tn + i % 4, so that lane l's accumulators hold, for x row l % 16
+  // of tile tm, the 4 TN consecutive columns from 4 TN (l / 16).
+  const int aoff[2] = {(wm0 + r16) * kARow + 16 * ((2 * h) ^ dma_aswz(r16)),
+                       (wm0 + r16) * kARow + 16 * ((2 * h + 1) ^ dma_aswz(r16))};
+  const int boff = kAStage + (wn0 + 4 * TN * (r16 / 4) + r16 % 4) * kBRow + 16 * (h ^ dma_bswz(r16 / 4));
 
-  f32x16 acc[TM][TN];
+  f32x4 acc[TM][TN];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
-    for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = f32x16{};
+    for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = f32x4{};
 
-  auto compute = [&](int stage) {
-    const char* sm = smem + stage * kDmaStage;
+  bf16x8 af[2][TM], bf[2][TN];
+  auto load_fragments = [&](const char* sm) {
+    u32x4 raw[TN];
 #pragma unroll
-    for (int p = 0; p < 2; ++p) {
-      bf16x8 bl[TN][2];
+    for (int tn = 0; tn < TN; ++tn) raw[tn] = *(const u32x4*)(sm + boff + tn * 4 * kBRow);
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) {
-        const u32x4 w16 = *(const u32x4*)(sm + brow + tn * 32 * kDmaBRow + bch[p]);
-        bl[tn][0] = int8x8_to_bf16(w16.x, w16.y);
-        bl[tn][1] = int8x8_to_bf16(w16.z, w16.w);
-      }
+    for (int u = 0; u < 2; ++u)
 #pragma unroll
-      for (int u = 0; u < 2; ++u) {
-        bf16x8 af[TM];
+      for (int tm = 0; tm < TM; ++tm) af[u][tm] = *(const bf16x8*)(sm + aoff[u] + tm * 16 * kARow);
 #pragma unroll
-        for (int tm = 0; tm < TM; ++tm) af[tm] = *(const bf16x8*)(sm + arow + tm * 32 * kDmaARow + ach[p][u]);
-#pragma unroll
-        for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-          for (int tn = 0; tn < TN; ++tn)
-            acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[tm], bl[tn][u], acc[tm][tn], 0, 0, 0);
-      }
+    for (int tn = 0; tn < TN; ++tn) {
+      bf[0][tn] = int8x8_to_bf16(raw[tn].x, raw[tn].y);
+      bf[1][tn] = int8x8_to_bf16(raw[tn].z, raw[tn].w);
     }
   };
+  auto mma = [&]() {
+    __builtin_amdgcn_s_setprio(1);
+#pragma unroll
+    for (int u = 1; u >= 0; --u)
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+          acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(bf[u][tn], af[u][tm], acc[tm][tn], 0, 0, 0);
+    __builtin_amdgcn_s_setprio(0);
+  };
+  auto phase_end = [&]() {
+    __builtin_amdgcn_sched_barrier(0);
+    lds_barrier();
+    __builtin_amdgcn_sched_barrier(0);
+  };
 
-  // Step kt: wait for this wavefront's loads of step kt (those of step kt + 1 may stay in flight), publish them
-  // with the barrier (which also retires every wavefront's reads of step kt - 1's stage), refill that stage with
-  // step kt + 2, multiply step kt.
   const int nk = a.K / kDmaBK;
+  const bool second = wave >= kDmaWaves / 2;
   issue(0, 0);
-  if (nk > 1) issue(1, 1);
+  if (nk > 1) {
+    issue(1, 1);
+    wait_steps(One{});
+  } else {
+    EGPT_WAIT_VMCNT(0);
+  }
+  lds_barrier();
+  if (second) lds_barrier();
   int stage = 0;
   for (int kt = 0; kt < nk; ++kt) {
-    if (kt + 1 < nk)
-      EGPT_WAIT_VMCNT(kDmaALoads + kDmaBLoads);
-    else
-      EGPT_WAIT_VMCNT(0);
-    lds_barrier();
+    const char* sm = smem + stage * kStage;
+    auto wait_next = [&]() {
+      if (kt + 2 < nk)
+        wait_steps(One{});
+      else
+        EGPT_WAIT_VMCNT(0);
+    };
     if (kt + 2 < nk) issue(kt + 2, stage == 0 ? 2 : stage - 1);
-    compute(stage);
-    stage = stage == 2 ? 0 : stage + 1;
+    load_fragments(sm);
+    if (second) wait_next();
+    phase_end();
+    mma();
+    if (!second) wait_next();
+    phase_end();
+    stage = stage == kDmaStages - 1 ? 0 : stage + 1;
   }
-  gemm_store<BM, BN, TM, TN, WN, SWIGLU>(a, acc, m0, n0, wm0, wn0, pid_n, lane, wave);
+  if (!second) lds_barrier();
+
+  if constexpr (SWIGLU) {
+    const int64_t f0 = (int64_t)pid_n * (BN / 2) + (wave % WN) * (8 * TN) + 2 * TN * h;
+    float gs[2 * TN], us[2 * TN];
+#pragma unroll
+    for (int e = 0; e < 2 * TN; ++e) {
+      const int64_t f = min(f0 + e, (int64_t)a.inter - 1);
+      gs[e] = a.scale[f];
+      us[e] = a.scale[a.inter + f];
+    }
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      const int64_t m = m0 + wm0 + 16 * tm + r16;
+      float o[2 * TN];
+#pragma unroll
+      for (int e = 0; e < 2 * TN; ++e) {
+        const float g = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][e / 4][e % 4])) * gs[e]));
+        const float u = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][TN / 2 + e / 4][e % 4])) * us[e]));
+        o[e] = bf16_to_f32(f32_to_bf16(g / (1.0f + expf(-g)))) * u;
+      }
+      store_row<2 * TN>(a, m, f0, a.inter, o);
+    }
+  } else {
+    const int64_t c0 = n0 + wn0 + 4 * TN * h;
+    float sc[4 * TN];
+#pragma unroll
+    for (int e = 0; e < 4 * TN; ++e) sc[e] = a.scale[min(c0 + e, (int64_t)a.N - 1)];
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      const int64_t m = m0 + wm0 + 16 * tm + r16;
+      float o[4 * TN];
+#pragma unroll
+      for (int e = 0; e < 4 * TN; ++e) o[e] = bf16_to_f32(f32_to_bf16(acc[tm][e / 4][e % 4])) * sc[e];
+      store_row<4 * TN>(a, m, c0, a.N, o);
+    }
+  }
 }
 
 // Split-K reduce: y[m, n] = bf16(bf16(sum_s part[s][m][n]) * scale[n]), splits added in order. The split
@@ -588,9 +587,12 @@ unsigned gemm_blocks(const GemmArgs& a) {
 
 constexpr int kMaxSplits = 16;
 
-// Tiles whose weights go to LDS as bf16 (converted once per block, int8_gemm_kernel's BF16B).
-template <int BM, int BN>
-constexpr bool kBf16B = (BM == 64 && BN == 64) || (BM == 128 && BN == 64) || (BM == 128 && BN == 128);
+// 128 x 128 tiles of a product from which the LDS-direct tiles take it. With fewer, most CUs would run one block's
+// chain of K steps alone (measured on the MI355X, us against the 64-row tiles: 144 tiles 300 x 4096 -> 6144 41.8 / 46.5,
+// 192 tiles 700 x 2048 -> 4096 23.4 / 27.7 and 130 x 2048 -> 12288 23.1 / 27.5, 256 tiles 1000 x 12288 -> 4096 126.1 /
+// 126.4; but 128 tiles 1000 x 2048 -> 2048 23.0 / 20.7 and 512 x 4096 -> 4096 41.7 / 34.4, 96 tiles 200 x 4096 -> 6144
+// 41.7 / 32.5).
+constexpr int kDmaMinTiles = 144;
 
 // The reduce for a.splits (2 ... S) slices; false for a count outside that range.
 template <int S>
@@ -610,7 +612,7 @@ int launch_split_partials(GemmArgs a, hipStream_t st) {
   a.tiles_m = (int)(((int64_t)a.M + 63) / 64);
   a.tiles_n = (int)(((int64_t)a.N + 63) / 64);
   const unsigned tiles = (unsigned)a.tiles_m * (unsigned)a.tiles_n;
-  hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, true, 2, 4, false, kBf16B<64, 64>>),
+  hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, true, 2, 4>),
                      dim3(tiles * (unsigned)a.splits), dim3(4 * kWave), 0, st, a);
   return EGPT_LAUNCH_STATUS();
 }
@@ -635,24 +637,70 @@ int launch_gemm(GemmArgs a, hipStream_t st) {
     // 16.5 -> 12.5 us, 160 x 2048 -> 4096 16.8 -> 13.2; with 320 tiles, 300 x 2048
     // -> 4096, 1.7% slower).
     if (a.K % kBKSplit == 0 && tiles < 256) {
-      hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, false, 2, 4, false, kBf16B<64, 64>>), dim3(tiles),
+      hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, false, 2, 4>), dim3(tiles),
                          dim3(4 * kWave), 0, st, a);
       return EGPT_LAUNCH_STATUS();
     }
   }
-  hipLaunchKernelGGL((int8_gemm_kernel<BM, BN, kBK, false, WN, NW, false, kBf16B<BM, BN>>), dim3(tiles),
+  hipLaunchKernelGGL((int8_gemm_kernel<BM, BN, kBK, false, WN, NW>), dim3(tiles),
                      dim3(NW * kWave), 0, st, a);
   return EGPT_LAUNCH_STATUS();
 }
 
-// The 256 x 256 LDS-direct tiles (K a multiple of 64); with SWIGLU each block covers 128 features.
-template <bool SWIGLU>
+// The LDS-direct tiles (K a multiple of 64); with SWIGLU each block covers 32 TN features.
+template <int TM, int TN, bool SWIGLU>
 int launch_gemm_dma(GemmArgs a, hipStream_t st) {
-  a.tiles_m = (int)(((int64_t)a.M + 255) / 256);
-  a.tiles_n = SWIGLU ? (int)(((int64_t)a.inter + 127) / 128) : (int)(((int64_t)a.N + 255) / 256);
-  hipLaunchKernelGGL((int8_gemm_dma_kernel<SWIGLU>), dim3((unsigned)a.tiles_m * (unsigned)a.tiles_n),
+  constexpr int BM = 32 * TM, BN = 64 * TN;
+  a.tiles_m = (int)(((int64_t)a.M + BM - 1) / BM);
+  a.tiles_n = SWIGLU ? (int)(((int64_t)a.inter + BN / 2 - 1) / (BN / 2)) : (int)(((int64_t)a.N + BN - 1) / BN);
+  hipLaunchKernelGGL((int8_gemm_dma_kernel<TM, TN, SWIGLU>), dim3((unsigned)a.tiles_m * (unsigned)a.tiles_n),
                      dim3(kDmaWaves * kWave), 0, st, a);
   return EGPT_LAUNCH_STATUS();
+}
+
+// Which LDS-direct tile: the least time of the launch's rounds of 256 blocks (one per CU; the 128 x 128 tile fits two
+// blocks on a CU, and a pair of them takes less than two rounds). The costs are the us of one full round over
+// K = 4096, launch excluded, measured on the MI355X; their ratios hold for other K.
+struct DmaTile {
+  int tm, tn;
+  float round;  // 256 blocks
+  float pair;   // 512 blocks, where two fit on a CU
+};
+constexpr DmaTile kDmaTiles[] = {{8, 4, 95.0f, 0.f}, {6, 4, 79.5f, 0.f}, {8, 3, 79.5f, 0.f}, {6, 3, 65.3f, 0.f},
+                                 {4, 4, 61.7f, 0.f}, {8, 2, 59.5f, 0.f}, {4, 3, 53.8f, 0.f}, {6, 2, 50.0f, 0.f},
+                                 {4, 2, 39.7f, 64.0f}};
+
+float dma_cost(const DmaTile& t, int64_t M, int64_t N) {
+  const int64_t tiles = ((M + 32 * t.tm - 1) / (32 * t.tm)) * ((N + 64 * t.tn - 1) / (64 * t.tn));
+  if (t.pair == 0.f) return t.round * (float)((tiles + 255) / 256);
+  const int64_t rest = tiles % 512;
+  return t.pair * (float)(tiles / 512) + (rest == 0 ? 0.f : rest <= 256 ? t.round : t.pair);
+}
+
+// N counts a SwiGLU product's gate and up columns; its tiles need an even TN.
+template <bool SWIGLU>
+int launch_gemm_dma_best(const GemmArgs& a, hipStream_t st) {
+  const DmaTile* best = nullptr;
+  for (const DmaTile& t : kDmaTiles)
+    if (!(SWIGLU && t.tn % 2) && (!best || dma_cost(t, a.M, a.N) < dma_cost(*best, a.M, a.N))) best = &t;
+  switch (best->tm * 8 + best->tn) {
+    case 8 * 8 + 4: return launch_gemm_dma<8, 4, SWIGLU>(a, st);
+    case 6 * 8 + 4: return launch_gemm_dma<6, 4, SWIGLU>(a, st);
+    case 4 * 8 + 4: return launch_gemm_dma<4, 4, SWIGLU>(a, st);
+    case 8 * 8 + 2: return launch_gemm_dma<8, 2, SWIGLU>(a, st);
+    case 6 * 8 + 2: return launch_gemm_dma<6, 2, SWIGLU>(a, st);
+    case 4 * 8 + 2: return launch_gemm_dma<4, 2, SWIGLU>(a, st);
+    default: break;
+  }
+  if constexpr (!SWIGLU) {
+    switch (best->tm * 8 + best->tn) {
+      case 8 * 8 + 3: return launch_gemm_dma<8, 3, false>(a, st);
+      case 6 * 8 + 3: return launch_gemm_dma<6, 3, false>(a, st);
+      case 4 * 8 + 3: return launch_gemm_dma<4, 3, false>(a, st);
+      default: break;
+    }
+  }
+  return EGPT_ERR_INVALID;
 }
 
 // The same product for shapes the MFMA kernel does not take (K not a multiple of
@@ -760,10 +808,9 @@ extern "C" int egpt_int8_gemm_ws(const void* x, int64_t ldx, const int8_t* w, in
       return launch_gemm<64, 64>(a, stream);
     }
   }
-// The largest tile that still gives every CU a block; small M keeps more, narrower tiles.
-  if (M > 128 && gemm_blocks<256, 256>(a) >= 256) return launch_gemm_dma<false>(a, stream);
-  if (M > 64 && gemm_blocks<128, 256>(a) >= 256) return launch_gemm<128, 256, kWN256, kNW256>(a, stream);
-  if (M > 64 && gemm_blocks<128, 128>(a) >= 256) return launch_gemm<128, 128, kWN128, kNW128>(a, stream);
+  // The LDS-direct tiles from kDmaMinTiles tiles of their smallest size; below, the 64-row tiles, whose more and
+  // shorter blocks fill more of the chip.
+  if (M > 64 && gemm_blocks<128, 128>(a) >= kDmaMinTiles) return launch_gemm_dma_best<false>(a, stream);
   if (M > 64 && gemm_blocks<128, 64>(a) >= 256) return launch_gemm<128, 64>(a, stream);
   return launch_gemm<64, 64>(a, stream);
 }
@@ -780,19 +827,8 @@ extern "C" int egpt_int8_gemm_swiglu(const void* x, int64_t ldx, const int8_t* w
     return EGPT_ERR_UNSUPPORTED;
   GemmArgs a{(const uint16_t*)x, ldx, w, ldw, scale, (uint16_t*)act, ld_act, M, (int)N, K, 0, 0, 1, K, nullptr,
              inter};
-  // The tiles whose wavefronts own two column tiles (a feature's gate and up in one lane), where the plain
-  // product would take them: 256 x 256 and 128 x 256 (each block covers BN / 2 features).
-  auto blocks = [&](int bm, int bn) {
-    return (int64_t)((M + bm - 1) / bm) * ((inter + bn / 2 - 1) / (bn / 2));
-  };
-  if (M > 128 && blocks(256, 256) >= 256) return launch_gemm_dma<true>(a, stream);
-  if (M > 64 && blocks(128, 256) >= 256) {
-    a.tiles_m = (M + 127) / 128;
-    a.tiles_n = (inter + 127) / 128;
-    hipLaunchKernelGGL((int8_gemm_kernel<128, 256, kBK, false, kWN256, kNW256, true>),
-                       dim3((unsigned)(a.tiles_m * a.tiles_n)), dim3(kNW256 * kWave), 0, stream, a);
-    return EGPT_LAUNCH_STATUS();
-  }
+  // The LDS-direct tiles where the plain product would take them.
+  if (M > 64 && gemm_blocks<128, 128>(a) >= kDmaMinTiles) return launch_gemm_dma_best<true>(a, stream);
   // 64 x 64 tiles (32 features each, gate and up in the two halves of a wavefront's tile) where the plain
   // product would run them too: not where it would split K, which this form cannot.
   int splits, kchunk;
@@ -802,10 +838,10 @@ extern "C" int egpt_int8_gemm_swiglu(const void* x, int64_t ldx, const int8_t* w
   a.tiles_n = (inter + 31) / 32;
   const unsigned tiles = (unsigned)a.tiles_m * (unsigned)a.tiles_n;
   if (K % kBKSplit == 0 && tiles < 256)
-    hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, false, 2, 4, true, kBf16B<64, 64>>), dim3(tiles),
+    hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, false, 2, 4, true>), dim3(tiles),
                        dim3(4 * kWave), 0, stream, a);
   else
-    hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBK, false, 2, 4, true, kBf16B<64, 64>>), dim3(tiles),
+    hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBK, false, 2, 4, true>), dim3(tiles),
                        dim3(4 * kWave), 0, stream, a);
   return EGPT_LAUNCH_STATUS();
 }

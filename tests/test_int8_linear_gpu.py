@@ -291,6 +291,49 @@ def test_prefill_gemm_kernel_matches_oracle(m, k, n):
     assert float((diff == 0).float().mean()) >= 0.9
 
 
+# 32 TM x 64 TN tiles of the LDS-direct kernel and shapes that take each: 1 to 4 K steps (the pipeline's prologue and
+# tail), ragged rows and features, an odd output pitch (stores off 16-byte alignment)
+DMA_TILE_SHAPES = [('4x2', 77, 192, 18441), ('6x2', 130, 64, 18440), ('4x3', 200, 128, 18443), ('4x4', 300, 256, 18440),
+                   ('8x2', 500, 192, 12300), ('6x4', 700, 192, 12300), ('8x4', 1000, 128, 12301),
+                   ('6x3', 1300, 192, 6150), ('8x3', 2500, 64, 14002)]
+
+
+@pytest.mark.parametrize('tile,m,k,n', DMA_TILE_SHAPES)
+def test_prefill_gemm_lds_direct_tiles_match_oracle(tile, m, k, n):
+    """Every tile of the LDS-direct GEMM against the oracle's prefill formula; rows and columns past the output stay
+    untouched."""
+    from efficientgpt_amd import _lib
+    x, q, s = make_case(m, k, n, seed=m + k + n)
+    xd, qd, sd = x.cuda(), q.cuda(), s.cuda()
+    y = torch.full((m + 1, n + 3), 7.0, device='cuda', dtype=torch.bfloat16)
+    st = _lib.lib().egpt_int8_gemm(xd.data_ptr(), k, qd.data_ptr(), k, sd.data_ptr(), y.data_ptr(), n + 3, m, n, k,
+                                   _lib.stream_ptr())
+    assert st == 0, st
+    check_against_oracle(y[:m, :n].cpu(), x, q, s)
+    assert bool((y[m] == 7).all()) and bool((y[:, n:] == 7).all())
+
+
+@pytest.mark.parametrize('tile,m,k,inter', [('4x2', 77, 192, 9221), ('6x2', 130, 64, 9220), ('8x2', 200, 128, 9223),
+                                            ('4x4', 300, 256, 9220), ('6x4', 1300, 192, 3075), ('8x4', 1000, 64, 6150)])
+def test_gemm_swiglu_lds_direct_tiles_match_the_two_calls(tile, m, k, inter):
+    """The SwiGLU form of every LDS-direct tile it has, bit for bit against the product followed by egpt_silu_mul."""
+    from efficientgpt_amd import _lib
+    lib = _lib.lib()
+    x, q, s = make_case(m, k, 2 * inter, seed=m + inter)
+    xd, qd, sd = x.cuda(), q.cuda(), s.cuda()
+    gu = torch.empty(m, 2 * inter, device='cuda', dtype=torch.bfloat16)
+    two = torch.empty(m, inter, device='cuda', dtype=torch.bfloat16)
+    one = torch.full((m, inter), float('nan'), device='cuda', dtype=torch.bfloat16)
+    st = _lib.stream_ptr()
+    assert lib.egpt_int8_gemm(xd.data_ptr(), k, qd.data_ptr(), k, sd.data_ptr(), gu.data_ptr(), 2 * inter, m,
+                              2 * inter, k, st) == 0
+    assert lib.egpt_silu_mul(gu.data_ptr(), 2 * inter, inter, two.data_ptr(), inter, m, st) == 0
+    assert lib.egpt_int8_gemm_swiglu(xd.data_ptr(), k, qd.data_ptr(), k, sd.data_ptr(), one.data_ptr(), inter, m,
+                                     inter, k, st) == 0
+    torch.cuda.synchronize()
+    assert torch.equal(one, two)
+
+
 SPLIT_SHAPES = [(128, 6144, 2048), (128, 2048, 4096), (33, 6144, 2048), (64, 2048, 2048), (100, 4096, 1000),
                 (17, 12288, 64), (200, 2048, 2048), (130, 2048, 2000), (256, 2048, 2048)]
 
