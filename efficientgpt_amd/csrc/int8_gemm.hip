@@ -9,12 +9,10 @@
 // GEMM; here the weights are converted on the chip, so they cross HBM once, as int8.
 //
 // Design:
-//   * Large products run tiles of 128 x 128 to 256 x 256 on v_mfma_f32_16x16x32_bf16 (int8_gemm_dma_kernel): operands
-//     straight into LDS, the weights as int8, eight wavefronts whose two halves take turns at the matrix cores.
-//   * Small ones run 64 x 64 and 128 x 64 tiles of 4 wavefronts on v_mfma_f32_32x32x16_bf16 (int8_gemm_kernel). K
-//     advances 64 (128 where the tiles are few) at a time through two LDS buffers and two register staging sets: the
-//     global loads of step k + 2 are issued before the MFMAs of step k; one barrier per step. The padding of the LDS
-//     rows puts the fragment reads of 16 consecutive rows on distinct banks.
+//   * Every tile runs v_mfma_f32_16x16x32_bf16 with its operands loaded straight into LDS, the weights as int8:
+//     128 x 128 to 256 x 256 for large products (int8_gemm_dma_kernel: eight wavefronts whose two halves take turns
+//     at the matrix cores), 32 x 64 to 128 x 64 for the others (int8_gemm_ring_kernel: more and shorter blocks).
+//     All sum an output in the same order, so its bits do not depend on the tile.
 //   * int8 -> bf16 is exact: every value in [-127, 127] is a bf16.
 //   * Rows past M or N read a valid row and are never stored.
 //   * Split-K (short M, long K: too few output tiles to give every CU a block):
@@ -22,9 +20,8 @@
 //     workspace [splits][M][N]; a second kernel adds the slices in split order and
 //     applies the two roundings. The fp32 sum is the same product in another
 //     order, as any GEMM blocking is.
-// Operand layouts of v_mfma_f32_32x32x16_bf16 (checked on the MI355X): lane l holds A[l % 32][8 (l / 32) + e]
-// and B[8 (l / 32) + e][l % 32], e = 0..7; accumulator register r of lane l is
-// C[8 (r / 4) + 4 (l / 32) + r % 4][l % 32].
+// Operand layouts of v_mfma_f32_16x16x32_bf16 (checked on the MI355X): lane l holds A[l % 16][8 (l / 16) + e]
+// and B[8 (l / 16) + e][l % 16], e = 0..7; accumulator register r of lane l is C[4 (l / 16) + r][l % 16].
 #include <algorithm>
 #include <type_traits>
 
@@ -34,24 +31,11 @@ namespace egpt {
 namespace {
 
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
-typedef float f32x16 __attribute__((ext_vector_type(16)));
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
 
-constexpr int kBK = 64;        // K per LDS stage of the one-pass kernel: K must be a multiple of it
-constexpr int kBKSplit = 128;  // K per LDS stage of the split-K slices (half the dependent steps)
-
-template <int BM, int BN, int BK, int WN, int NW>
-struct GemmShape {
-  static constexpr int NT = NW * kWave;      // threads of the block
-  static constexpr int WM = NW / WN;          // wavefronts along M (the block's NW as WM x WN)
-  static constexpr int TM = BM / (32 * WM);  // 32 x 32 tiles per wavefront along M
-  static constexpr int TN = BN / (32 * WN);  // ... along N
-  static constexpr int kLdsRow = BK + 8;    // bf16 elements per x or weight row in LDS (16 bytes of padding)
-  static constexpr int kALoads = BM * BK * 2 / (NT * 16);  // 16-byte x loads per thread per step
-  static constexpr int kBLoads = BN * BK / (NT * 16);      // 16-byte int8 loads per thread per step
-  static_assert(WM * WN == NW && TM >= 1 && TN >= 1 && kALoads >= 1 && kBLoads >= 1, "tile too small for the block");
-};
+constexpr int kBK = 64;        // K must be a multiple of it
+constexpr int kBKSplit = 128;  // K slices of a split are multiples of it
 
 // 8 int8 (one LDS fragment) -> 8 bf16, exact.
 __device__ __forceinline__ bf16x8 int8x8_to_bf16(const uint32_t w0, const uint32_t w1) {
@@ -85,16 +69,6 @@ struct GemmArgs {
   int inter;           // SwiGLU form: features (w holds inter gate rows, then inter up rows; N = 2 inter)
 };
 
-// SwiGLU form of the small tiles: block tile column j (of BN) -> weight row. Each wavefront's BN / WN columns hold its
-// features' gate rows and then the same features' up rows. Features past `inter` read the last one.
-template <int BN, int WN>
-__device__ __forceinline__ int64_t swiglu_row(int64_t pid_n, int j, int inter) {
-  constexpr int kPerWave = BN / WN, kHalf = kPerWave / 2;
-  const int wn = j / kPerWave, o = j % kPerWave;
-  const int64_t f = min(pid_n * (BN / 2) + wn * kHalf + (o % kHalf), (int64_t)inter - 1);
-  return o < kHalf ? f : inter + f;
-}
-
 constexpr int kXcds = 8;        // MI355X: 8 XCDs, each with its own L2
 constexpr int kGroupM = 8;      // M tiles per group of the tile order
 
@@ -115,211 +89,6 @@ __device__ __forceinline__ void gemm_tile(int b, int tiles_m, int tiles_n, int& 
   const int gm = min(tiles_m - first_m, kGroupM);
   pid_m = first_m + (t % group) % gm;
   pid_n = (t % group) / gm;
-}
-
-// The store of a block's accumulators (TM x TN 32 x 32 tiles per wavefront, wavefront tile origin wm0, wn0 in the
-// block tile m0, n0): y = bf16(bf16(acc) * scale), the reference's two roundings, or with SWIGLU the activation
-// of each feature from its gate and up columns.
-template <int BM, int BN, int TM, int TN, int WN, bool SWIGLU>
-__device__ __forceinline__ void gemm_store(const GemmArgs& a, const f32x16 (&acc)[TM][TN], int64_t m0, int64_t n0,
-                                           int wm0, int wn0, int pid_n, int lane, int wave) {
-  // y = bf16(bf16(acc) * scale): the reference's two roundings. Stores address y
-  // by 32-bit byte offsets from the row of this lane's first accumulator (the
-  // host checks that y spans < 2 GiB); row r of a tile is a constant multiple of
-  // the row pitch away.
-  char* yb = (char*)a.y;
-  const int64_t mrow0 = m0 + wm0 + 4 * (lane / 32);
-  const uint32_t pitch = (uint32_t)(a.ldy * 2);
-  if constexpr (SWIGLU && TN == 1) {
-    // One 32-column tile per wavefront: its columns 0-15 are the gate rows of 16 features and 16-31 their up
-    // rows (swiglu_row), so lane l (column l % 32 < 16) takes u from lane l ^ 16, the same rows one tile half
-    // over. The arithmetic per element is the form below.
-    const int c = lane % 32;
-    const int64_t f = (int64_t)pid_n * (BN / 2) + (wave % WN) * (BN / WN / 2) + (c % 16);
-    const int64_t fc = min(f, (int64_t)a.inter - 1);
-    const float sg_scale = a.scale[fc], su_scale = a.scale[a.inter + fc];
-    const uint32_t base = (uint32_t)((mrow0 * a.ldy + f) * 2);
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const float up = __shfl_xor(acc[tm][0][r], 16);
-        const int dm = tm * 32 + 8 * (r / 4) + r % 4;
-        if (c < 16 && mrow0 + dm < a.M && f < a.inter) {
-          const float g = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][0][r])) * sg_scale));
-          const float u = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(up)) * su_scale));
-          const float sg = bf16_to_f32(f32_to_bf16(g / (1.0f + expf(-g))));
-          *(uint16_t*)(yb + (base + (uint32_t)dm * pitch)) = f32_to_bf16(sg * u);
-        }
-      }
-    }
-    return;
-  }
-#pragma unroll
-  for (int tn = 0; tn < TN; ++tn) {
-    const int64_t n = n0 + wn0 + tn * 32 + lane % 32;
-    const float sc = a.scale[min(n, (int64_t)a.N - 1)];
-    const uint32_t base = (uint32_t)((mrow0 * a.ldy + n) * 2);
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-#pragma unroll
-      for (int r = 0; r < 16; ++r) {
-        const int dm = tm * 32 + 8 * (r / 4) + r % 4;
-        if (mrow0 + dm < a.M && n < a.N) {
-          const float v = bf16_to_f32(f32_to_bf16(acc[tm][tn][r]));
-          *(uint16_t*)(yb + (base + (uint32_t)dm * pitch)) = f32_to_bf16(v * sc);
-        }
-      }
-    }
-  }
-}
-
-// The small tiles (64 x 64 and 128 x 64): the weights are converted to bf16 once, by the thread that loaded them, as
-// they are written to LDS, and the wavefronts read bf16 fragments.
-template <int BM, int BN, int BK, bool SPLIT, int WN, int NW, bool SWIGLU = false>
-__global__ __launch_bounds__(NW * kWave, 1) void int8_gemm_kernel(const GemmArgs a) {
-  using S = GemmShape<BM, BN, BK, WN, NW>;
-  constexpr int TM = S::TM, TN = S::TN;
-  static_assert(!SWIGLU || (!SPLIT && TN == 1), "the SwiGLU form pairs the two halves of a wavefront's one column tile");
-  constexpr int kLdsRow = S::kLdsRow;
-  __shared__ __align__(16) uint16_t As[2][BM * kLdsRow];
-  __shared__ __align__(16) uint16_t Bs[2][BN * kLdsRow];
-
-  const int tid = threadIdx.x;
-  const int lane = tid & (kWave - 1);
-  const int wave = tid / kWave;
-  const int wm0 = (wave / WN) * (BM / S::WM);  // wavefront tile origin in the block tile
-  const int wn0 = (wave % WN) * (BN / WN);
-  const int tiles = a.tiles_m * a.tiles_n;
-  const int split = SPLIT ? (int)blockIdx.x / tiles : 0;
-  int pid_m, pid_n;
-  gemm_tile((int)blockIdx.x - split * tiles, a.tiles_m, a.tiles_n, pid_m, pid_n);
-  const int64_t m0 = (int64_t)pid_m * BM;
-  const int64_t n0 = (int64_t)pid_n * BN;
-  const int kbeg = SPLIT ? split * a.kchunk : 0;  // this block's K slice [kbeg, kbeg + nk * BK)
-
-  // global -> register staging of one K step: 32-bit byte offsets from the
-  // operands' base pointers (the host checks that both operands span < 2 GiB)
-  const char* xb = (const char*)a.x;
-  const char* wb = (const char*)a.w;
-  uint32_t xoff[S::kALoads];
-  int a_lds[S::kALoads];
-#pragma unroll
-  for (int j = 0; j < S::kALoads; ++j) {
-    const int i = tid + j * S::NT;
-    const int row = i / (BK / 8), chunk = i % (BK / 8);
-    xoff[j] = (uint32_t)((min(m0 + row, (int64_t)a.M - 1) * a.ldx + kbeg + chunk * 8) * 2);
-    a_lds[j] = row * kLdsRow + chunk * 8;
-  }
-  uint32_t woff[S::kBLoads];
-  int b_lds[S::kBLoads];
-#pragma unroll
-  for (int j = 0; j < S::kBLoads; ++j) {
-    const int i = tid + j * S::NT;
-    const int row = i / (BK / 16), chunk = i % (BK / 16);
-    const int64_t wrow = SWIGLU ? swiglu_row<BN, WN>(pid_n, row, a.inter) : min(n0 + row, (int64_t)a.N - 1);
-    woff[j] = (uint32_t)(wrow * a.ldw + kbeg + chunk * 16);
-    b_lds[j] = row * kLdsRow + chunk * 16;
-  }
-  // Two register staging sets: the loads of step k + 2 are issued while step k is
-  // multiplied and land in LDS among the MFMAs of step k + 1, one to two steps of
-  // MFMA work later. Loads past the last step re-read the last K slice (in bounds, never
-  // stored), so every load is unconditional and each wait is for one set only.
-  const int nk = (SPLIT ? min(a.kchunk, a.K - kbeg) : a.K) / BK;
-  u32x4 xr[2][S::kALoads], wr[2][S::kBLoads];
-  auto load_step = [&](int kt, int set) {
-    const uint32_t k0 = (uint32_t)(min(kt, nk - 1) * BK);
-#pragma unroll
-    for (int j = 0; j < S::kALoads; ++j) xr[set][j] = ld16(xb + (xoff[j] + 2 * k0));
-#pragma unroll
-    for (int j = 0; j < S::kBLoads; ++j) wr[set][j] = ld16_stream(wb + (woff[j] + k0));
-  };
-  auto store_step = [&](int buf, int set) {
-#pragma unroll
-    for (int j = 0; j < S::kALoads; ++j) *(u32x4*)&As[buf][a_lds[j]] = xr[set][j];
-#pragma unroll
-    for (int j = 0; j < S::kBLoads; ++j) {
-      *(bf16x8*)&Bs[buf][b_lds[j]] = int8x8_to_bf16(wr[set][j].x, wr[set][j].y);
-      *(bf16x8*)&Bs[buf][b_lds[j] + 8] = int8x8_to_bf16(wr[set][j].z, wr[set][j].w);
-    }
-  };
-
-  f32x16 acc[TM][TN];
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = f32x16{};
-
-  // fragment offsets (elements) inside one LDS buffer
-  const int frag_k = 8 * (lane / 32);
-  int a_frag[TM], b_frag[TN];
-#pragma unroll
-  for (int tm = 0; tm < TM; ++tm) a_frag[tm] = (wm0 + tm * 32 + lane % 32) * kLdsRow + frag_k;
-#pragma unroll
-  for (int tn = 0; tn < TN; ++tn) b_frag[tn] = (wn0 + tn * 32 + lane % 32) * kLdsRow + frag_k;
-
-  // The MFMAs of one K step from LDS buffer `buf`, then, with sbuf >= 0, the next step's LDS stores (staging set `set`
-  // into buffer sbuf). One wavefront per SIMD with a short MFMA chain per 16 columns leaves nothing to cover an LDS
-  // read issued just before its MFMA, so every fragment of the step is read first.
-  auto mma_step = [&](int buf, int sbuf = -1, int set = 0) {
-    bf16x8 af[BK / 16][TM], bh[BK / 16][TN];
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks) {
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm) af[ks][tm] = *(const bf16x8*)&As[buf][a_frag[tm] + ks * 16];
-#pragma unroll
-      for (int tn = 0; tn < TN; ++tn) bh[ks][tn] = *(const bf16x8*)&Bs[buf][b_frag[tn] + ks * 16];
-    }
-#pragma unroll
-    for (int ks = 0; ks < BK / 16; ++ks)
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int tn = 0; tn < TN; ++tn)
-          acc[tm][tn] = __builtin_amdgcn_mfma_f32_32x32x16_bf16(af[ks][tm], bh[ks][tn], acc[tm][tn], 0, 0, 0);
-    if (sbuf >= 0) store_step(sbuf, set);
-  };
-
-  load_step(0, 0);
-  load_step(1, 1);
-  store_step(0, 0);
-  __syncthreads();
-  // Pairs of steps so the staging sets are fixed registers: step kt computes LDS
-  // buffer kt & 1, refills set kt & 1 with step kt + 2 and stores set (kt + 1) & 1
-  // into the other buffer among its MFMAs; an odd last step runs after the loop. Scheduling barriers keep each phase in
-  // place (hoisting the second step's fragment reads above the first step's MFMAs
-  // would double the live registers).
-  int kt = 0;
-  for (; kt + 1 < nk; kt += 2) {
-    load_step(kt + 2, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    mma_step(0, 1, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    __syncthreads();
-    load_step(kt + 3, 1);
-    __builtin_amdgcn_sched_barrier(0);
-    mma_step(1, kt + 2 < nk ? 0 : -1, 0);
-    __builtin_amdgcn_sched_barrier(0);
-    if (kt + 2 < nk) __syncthreads();
-  }
-  if (kt < nk) mma_step(0);
-
-  if constexpr (SPLIT) {  // the fp32 tile of this K slice; the reduce kernel rounds
-    float* part = a.part + (int64_t)split * a.M * a.N;
-#pragma unroll
-    for (int tn = 0; tn < TN; ++tn) {
-      const int64_t n = n0 + wn0 + tn * 32 + lane % 32;
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-          const int64_t m = m0 + wm0 + tm * 32 + 8 * (r / 4) + 4 * (lane / 32) + r % 4;
-          if (m < a.M && n < a.N) part[m * a.N + n] = acc[tm][tn][r];
-        }
-    }
-    return;
-  }
-  gemm_store<BM, BN, TM, TN, WN, SWIGLU>(a, acc, m0, n0, wm0, wn0, pid_n, lane, wave);
 }
 
 // The large tiles: 32 TM x 64 TN of y per block, eight wavefronts as 2 (M) x 4 (N) of 16 TM x 16 TN each.
@@ -354,6 +123,8 @@ __device__ __forceinline__ int dma_bswz(int t) { return ((t & 1) << 1) ^ (3 * ((
 
 typedef uint32_t u32x4_h __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_h __attribute__((ext_vector_type(2), aligned(2)));
+typedef uint32_t u32_h __attribute__((aligned(2)));
+typedef float f32x4_w __attribute__((ext_vector_type(4), aligned(4)));
 
 // C consecutive outputs of row m from column c0, rounded to bf16: 16- and 8-byte stores at any element alignment, or one
 // by one where the row ends among them.
@@ -368,12 +139,51 @@ __device__ __forceinline__ void store_row(const GemmArgs& a, int64_t m, int64_t 
 #pragma unroll
     for (int i = 0; i + 4 <= C / 2; i += 4)
       *(global_ptr<u32x4_h>)(p + 2 * i) = u32x4{w[i], w[i + 1], w[i + 2], w[i + 3]};
-    if constexpr (C % 8)
-      *(global_ptr<u32x2_h>)(p + C - 4) = u32x2{w[C / 2 - 2], w[C / 2 - 1]};
+    if constexpr (C % 8 == 4) *(global_ptr<u32x2_h>)(p + C - 4) = u32x2{w[C / 2 - 2], w[C / 2 - 1]};
+    if constexpr (C % 8 == 2) *(global_ptr<u32_h>)(p + C - 2) = w[C / 2 - 1];
   } else {
 #pragma unroll
     for (int i = 0; i < C; ++i)
       if (c0 + i < cols) gstore(p + i, f32_to_bf16(o[i]));
+  }
+}
+
+// The store of a wavefront's accumulators in the 16x16x32 layout: lane l holds, for rows m, m + 16, ..., the 4 TN
+// consecutive columns from c0; y = bf16(bf16(acc) * scale), the reference's two roundings, or with SWIGLU the activation
+// of the 2 TN features from c0 (their gate columns, then their up columns).
+template <int TM, int TN, bool SWIGLU>
+__device__ __forceinline__ void gemm_store_rows(const GemmArgs& a, const f32x4 (&acc)[TM][TN], int64_t m, int64_t c0) {
+  if constexpr (SWIGLU) {
+    float gs[2 * TN], us[2 * TN];
+#pragma unroll
+    for (int e = 0; e < 2 * TN; ++e) {
+      const int64_t f = min(c0 + e, (int64_t)a.inter - 1);
+      gs[e] = a.scale[f];
+      us[e] = a.scale[a.inter + f];
+    }
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      float o[2 * TN];
+#pragma unroll
+      for (int e = 0; e < 2 * TN; ++e) {
+        const int v = 2 * TN + e;
+        const float g = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][e / 4][e % 4])) * gs[e]));
+        const float u = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][v / 4][v % 4])) * us[e]));
+        o[e] = bf16_to_f32(f32_to_bf16(g / (1.0f + expf(-g)))) * u;
+      }
+      store_row<2 * TN>(a, m + 16 * tm, c0, a.inter, o);
+    }
+  } else {
+    float sc[4 * TN];
+#pragma unroll
+    for (int e = 0; e < 4 * TN; ++e) sc[e] = a.scale[min(c0 + e, (int64_t)a.N - 1)];
+#pragma unroll
+    for (int tm = 0; tm < TM; ++tm) {
+      float o[4 * TN];
+#pragma unroll
+      for (int e = 0; e < 4 * TN; ++e) o[e] = bf16_to_f32(f32_to_bf16(acc[tm][e / 4][e % 4])) * sc[e];
+      store_row<4 * TN>(a, m + 16 * tm, c0, a.N, o);
+    }
   }
 }
 
@@ -520,40 +330,198 @@ __global__ __launch_bounds__(kDmaWaves * kWave, 1) void int8_gemm_dma_kernel(con
   }
   if (!second) lds_barrier();
 
-  if constexpr (SWIGLU) {
-    const int64_t f0 = (int64_t)pid_n * (BN / 2) + (wave % WN) * (8 * TN) + 2 * TN * h;
-    float gs[2 * TN], us[2 * TN];
+  gemm_store_rows<TM, TN, SWIGLU>(a, acc, m0 + wm0 + r16, (int64_t)pid_n * (SWIGLU ? BN / 2 : BN) +
+                                  (wave % WN) * (SWIGLU ? 8 * TN : 16 * TN) + (SWIGLU ? 2 : 4) * TN * h);
+}
+
+// The small tiles: BM x BN of y per block (16 TM x 16 TN per wavefront, WM x WN wavefronts), for products with too few
+// large tiles to fill the chip. Operands go straight into LDS as in int8_gemm_dma_kernel, 128 K columns a step through a
+// ring of STAGES; a wavefront reads a step's fragments into registers while it multiplies the step before, one barrier a
+// step. Each output is summed in the order of the large tiles (two MFMAs per 64 columns, the second half's first).
+//
+// What bounds it is LDS: at 300 x 12288 -> 4096 (96 x 64 tiles, one round of 256 blocks, 96 steps) the loads alone take
+// 43 us, the reads, conversions and MFMAs alone 29, together 64; the loads' distance (2 to 4 steps) and row slices of
+// 256 columns made no difference. Each x row is read from LDS by WN wavefronts and each weight row by WM, so eight
+// wavefronts as 2 x 4 did better than 4 x 2 (6-8%) or four (8-15%, too few to hide a barrier). It replaced 64 x 64 and
+// 128 x 64 tiles staged through registers, on the MI355X with the weights out of cache (us): 20 x 4096 -> 24576 SwiGLU
+// 36 -> 26, 77 x 2048 -> 12288 SwiGLU 20.4 -> 14.2, 200 x 4096 -> 6144 31.6 -> 26.7, 300 x 12288 -> 4096 97 -> 64, 300 x
+// 4096 -> 6144 42.5 -> 30, 600 x 2048 -> 2048 18.8 -> 13.1, 600 x 6144 -> 2048 51 -> 32.5; split slices 20 x 12288 ->
+// 4096 18.5 -> 16.5, at 64-128 rows within 3%.
+constexpr int kRingBK = 128;
+
+// LDS positions of a stage's 16-byte chunks: chunk c of x row r (16 a row) sits at c ^ (r & 15), chunk c of the weight
+// row that is slot i of its MFMA operand (8 a row) at c ^ (i >> 1): the 16 lanes that a 16-byte LDS read serves together
+// (see dma_bswz) fall on distinct banks.
+template <int TN>
+__device__ __forceinline__ int ring_slot(int row) { return (row / (4 * TN)) % 4 * 4 + row % 4; }
+
+template <int BM, int BN, int WM, int WN, int STAGES, bool SPLIT, bool SWIGLU>
+__global__ __launch_bounds__(WM * WN * kWave) void int8_gemm_ring_kernel(const GemmArgs a) {
+  constexpr int NW = WM * WN, TM = BM / (16 * WM), TN = BN / (16 * WN);
+  constexpr int kARow = kRingBK * 2, kBRow = kRingBK;  // bytes per x row / weight row of a stage
+  constexpr int kAStage = BM * kARow, kStage = kAStage + BN * kBRow;
+  constexpr int kALoads = kAStage / (NW * 1024), kBLoads = BN * kBRow / (NW * 1024);  // 1 KiB loads per wavefront
+  constexpr int kLoads = kALoads + kBLoads;
+  static_assert(kALoads * NW * 1024 == kAStage && kBLoads * NW * 1024 == BN * kBRow && TM >= 1 && TN >= 1, "");
+  static_assert(!(SPLIT && SWIGLU) && STAGES >= 2 && (STAGES - 1) * kLoads < 64, "");
+  __shared__ __align__(16) char smem[STAGES * kStage];
+
+  const int tid = threadIdx.x;
+  const int lane = tid & (kWave - 1);
+  const int wave = __builtin_amdgcn_readfirstlane(tid / kWave);
+  const int wm0 = (wave / WN) * (16 * TM);
+  const int wn0 = (wave % WN) * (16 * TN);
+  const int tiles = a.tiles_m * a.tiles_n;
+  const int split = SPLIT ? (int)blockIdx.x / tiles : 0;
+  int pid_m, pid_n;
+  gemm_tile((int)blockIdx.x - split * tiles, a.tiles_m, a.tiles_n, pid_m, pid_n);
+  const int64_t m0 = (int64_t)pid_m * BM;
+  const int64_t n0 = (int64_t)pid_n * BN;
+  const int kbeg = SPLIT ? split * a.kchunk : 0;
+  const int klen = SPLIT ? min(a.kchunk, a.K - kbeg) : a.K;  // a multiple of 64
+  const int nk = (klen + kRingBK - 1) / kRingBK;
+
+  // 32-bit byte offsets from the operands' bases (the host checks that both span < 2 GiB); rows past M or N read the
+  // last one, columns past the slice (a last step of 64) its last 16 bytes.
+  constexpr int kAC = kRingBK / 8, kBC = kRingBK / 16;  // chunks per row
+  uint32_t xr[kALoads], xc[kALoads], wr[kBLoads], wc[kBLoads];  // row offset, column offset in a step
 #pragma unroll
-    for (int e = 0; e < 2 * TN; ++e) {
-      const int64_t f = min(f0 + e, (int64_t)a.inter - 1);
-      gs[e] = a.scale[f];
-      us[e] = a.scale[a.inter + f];
+  for (int q = 0; q < kALoads; ++q) {
+    const int row = (wave * kALoads + q) * (64 / kAC) + lane / kAC;
+    xc[q] = 16 * ((lane % kAC) ^ (row & 15));
+    xr[q] = (uint32_t)((min(m0 + row, (int64_t)a.M - 1) * a.ldx + kbeg) * 2);
+  }
+#pragma unroll
+  for (int q = 0; q < kBLoads; ++q) {
+    const int row = (wave * kBLoads + q) * (64 / kBC) + lane / kBC;
+    wc[q] = 16 * ((lane % kBC) ^ (ring_slot<TN>(row) >> 1));
+    int64_t wrow;
+    if constexpr (SWIGLU) {  // each lane's 4 TN columns are 2 TN features' gate rows, then their up rows
+      const int o = row % (4 * TN);
+      const int64_t f = min((int64_t)pid_n * (BN / 2) + row / (4 * TN) * (2 * TN) + o % (2 * TN), (int64_t)a.inter - 1);
+      wrow = o < 2 * TN ? f : a.inter + f;
+    } else {
+      wrow = min(n0 + row, (int64_t)a.N - 1);
     }
+    wr[q] = (uint32_t)(wrow * a.ldw + kbeg);
+  }
+  const uint32_t sbase = lds_addr(smem);
+  const uint32_t xlim = (uint32_t)(2 * klen - 16), wlim = (uint32_t)(klen - 16);
+  auto issue = [&](int kt, int stage) {
+    const uint32_t abase = sbase + (uint32_t)(stage * kStage);
+#pragma unroll
+    for (int q = 0; q < kBLoads; ++q)
+      lds_load16_at(abase + (uint32_t)(kAStage + (wave * kBLoads + q) * 1024), a.w,
+                    wr[q] + min(wc[q] + (uint32_t)(kt * kBRow), wlim));
+#pragma unroll
+    for (int q = 0; q < kALoads; ++q)
+      lds_load16_at(abase + (uint32_t)((wave * kALoads + q) * 1024), a.x,
+                    xr[q] + min(xc[q] + (uint32_t)(kt * kARow), xlim));
+  };
+
+  const int r16 = lane % 16, h = lane / 16;
+  const int arow = (wm0 + r16) * kARow;
+  const int brow = kAStage + (wn0 + 4 * TN * (r16 / 4) + r16 % 4) * kBRow;
+  f32x4 acc[TM][TN];
+#pragma unroll
+  for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = f32x4{};
+  struct Frags {
+    u32x4 w[kRingBK / 64][TN];
+    bf16x8 x[kRingBK / 64][2][TM];
+  };
+  auto read = [&](Frags& f, const char* sm) {
+#pragma unroll
+    for (int s = 0; s < kRingBK / 64; ++s) {
+#pragma unroll
+      for (int tn = 0; tn < TN; ++tn)
+        f.w[s][tn] = *(const u32x4*)(sm + brow + tn * 4 * kBRow + 16 * ((4 * s + h) ^ (r16 >> 1)));
+#pragma unroll
+      for (int u = 1; u >= 0; --u)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+          f.x[s][u][tm] = *(const bf16x8*)(sm + arow + tm * 16 * kARow + 16 * ((8 * s + 2 * h + u) ^ r16));
+    }
+  };
+  auto mma = [&](const Frags& f, int s) {  // 64 columns
+    bf16x8 w[2][TN];
+#pragma unroll
+    for (int tn = 0; tn < TN; ++tn) {
+      w[1][tn] = int8x8_to_bf16(f.w[s][tn].z, f.w[s][tn].w);
+      w[0][tn] = int8x8_to_bf16(f.w[s][tn].x, f.w[s][tn].y);
+    }
+#pragma unroll
+    for (int u = 1; u >= 0; --u)
+#pragma unroll
+      for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+        for (int tn = 0; tn < TN; ++tn)
+          acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(w[u][tn], f.x[s][u][tm], acc[tm][tn], 0, 0, 0);
+  };
+  // Wait until no more than the loads of `later` steps are in flight, then publish what has arrived.
+  auto arrive = [&](int later) {
+    if (later >= STAGES - 1)
+      EGPT_WAIT_VMCNT((STAGES - 1) * kLoads);
+    else if (later == STAGES - 2)
+      EGPT_WAIT_VMCNT((STAGES - 2) * kLoads);
+    else if (STAGES > 3 && later == STAGES - 3)
+      EGPT_WAIT_VMCNT((STAGES > 3 ? STAGES - 3 : 0) * kLoads);
+    else
+      EGPT_WAIT_VMCNT(0);
+    lds_barrier();
+  };
+  // Step kt: the fragments of step kt + 1 are read while those of step kt, in registers, are multiplied. The barrier
+  // publishes stage kt + 1 and tells that every wavefront has read stage kt, whose buffer takes step kt + STAGES.
+  int stage = 0;
+  auto step = [&](int kt, const Frags& cur, Frags& next) {
+    const int ahead = stage == STAGES - 1 ? 0 : stage + 1;
+    if (kt + 1 < nk) {
+      arrive(min(STAGES - 2, nk - 2 - kt));
+      read(next, smem + ahead * kStage);
+    }
+    __builtin_amdgcn_sched_barrier(0);
+    if (kt + STAGES < nk) issue(kt + STAGES, stage);
+    __builtin_amdgcn_sched_barrier(0);
+    mma(cur, 0);
+    if (kt * kRingBK + 64 < klen) mma(cur, 1);
+    __builtin_amdgcn_sched_barrier(0);
+    stage = ahead;
+  };
+
+#pragma unroll
+  for (int s = 0; s < STAGES; ++s)
+    if (s < nk) issue(s, s);
+  Frags f0, f1;
+  arrive(min(STAGES - 1, nk - 1));
+  read(f0, smem);
+  for (int kt = 0; kt < nk; kt += 2) {
+    step(kt, f0, f1);
+    if (kt + 1 < nk) step(kt + 1, f1, f0);
+  }
+
+  if constexpr (SPLIT) {  // the fp32 tile of this K slice; the reduce kernel rounds
+    float* part = a.part + (int64_t)split * a.M * a.N;
+    const int64_t c0 = n0 + wn0 + 4 * TN * h;
 #pragma unroll
     for (int tm = 0; tm < TM; ++tm) {
       const int64_t m = m0 + wm0 + 16 * tm + r16;
-      float o[2 * TN];
+      if (m >= a.M) continue;
 #pragma unroll
-      for (int e = 0; e < 2 * TN; ++e) {
-        const float g = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][e / 4][e % 4])) * gs[e]));
-        const float u = bf16_to_f32(f32_to_bf16(bf16_to_f32(f32_to_bf16(acc[tm][TN / 2 + e / 4][e % 4])) * us[e]));
-        o[e] = bf16_to_f32(f32_to_bf16(g / (1.0f + expf(-g)))) * u;
+      for (int tn = 0; tn < TN; ++tn) {
+        float* p = part + m * a.N + c0 + 4 * tn;
+        if (c0 + 4 * tn + 4 <= a.N) {
+          *(global_ptr<f32x4_w>)p = acc[tm][tn];
+        } else {
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (c0 + 4 * tn + r < a.N) gstore(p + r, (float)acc[tm][tn][r]);
+        }
       }
-      store_row<2 * TN>(a, m, f0, a.inter, o);
     }
   } else {
-    const int64_t c0 = n0 + wn0 + 4 * TN * h;
-    float sc[4 * TN];
-#pragma unroll
-    for (int e = 0; e < 4 * TN; ++e) sc[e] = a.scale[min(c0 + e, (int64_t)a.N - 1)];
-#pragma unroll
-    for (int tm = 0; tm < TM; ++tm) {
-      const int64_t m = m0 + wm0 + 16 * tm + r16;
-      float o[4 * TN];
-#pragma unroll
-      for (int e = 0; e < 4 * TN; ++e) o[e] = bf16_to_f32(f32_to_bf16(acc[tm][e / 4][e % 4])) * sc[e];
-      store_row<4 * TN>(a, m, c0, a.N, o);
-    }
+    gemm_store_rows<TM, TN, SWIGLU>(a, acc, m0 + wm0 + r16, (int64_t)pid_n * (SWIGLU ? BN / 2 : BN) +
+                                    (wave % WN) * (SWIGLU ? 8 * TN : 16 * TN) + (SWIGLU ? 2 : 4) * TN * h);
   }
 }
 
@@ -580,19 +548,7 @@ __global__ __launch_bounds__(kReduceThreads) void int8_gemm_reduce_kernel(const 
   }
 }
 
-template <int BM, int BN>
-unsigned gemm_blocks(const GemmArgs& a) {
-  return (unsigned)(((int64_t)a.N + BN - 1) / BN) * (unsigned)(((int64_t)a.M + BM - 1) / BM);
-}
-
 constexpr int kMaxSplits = 16;
-
-// 128 x 128 tiles of a product from which the LDS-direct tiles take it. With fewer, most CUs would run one block's
-// chain of K steps alone (measured on the MI355X, us against the 64-row tiles: 144 tiles 300 x 4096 -> 6144 41.8 / 46.5,
-// 192 tiles 700 x 2048 -> 4096 23.4 / 27.7 and 130 x 2048 -> 12288 23.1 / 27.5, 256 tiles 1000 x 12288 -> 4096 126.1 /
-// 126.4; but 128 tiles 1000 x 2048 -> 2048 23.0 / 20.7 and 512 x 4096 -> 4096 41.7 / 34.4, 96 tiles 200 x 4096 -> 6144
-// 41.7 / 32.5).
-constexpr int kDmaMinTiles = 144;
 
 // The reduce for a.splits (2 ... S) slices; false for a count outside that range.
 template <int S>
@@ -607,49 +563,33 @@ bool launch_reduce(const GemmArgs& a, unsigned blocks, hipStream_t st) {
   }
 }
 
-// The split slices' fp32 tiles into a.part (64 x 64 tiles, a.splits > 1); no reduce.
-int launch_split_partials(GemmArgs a, hipStream_t st) {
-  a.tiles_m = (int)(((int64_t)a.M + 63) / 64);
-  a.tiles_n = (int)(((int64_t)a.N + 63) / 64);
-  const unsigned tiles = (unsigned)a.tiles_m * (unsigned)a.tiles_n;
-  hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, true, 2, 4>),
-                     dim3(tiles * (unsigned)a.splits), dim3(4 * kWave), 0, st, a);
-  return EGPT_LAUNCH_STATUS();
-}
-
-template <int BM, int BN, int WN = 2, int NW = 4>
-int launch_gemm(GemmArgs a, hipStream_t st) {
+template <int BM, int BN, int WM, int WN, int STAGES, bool SPLIT, bool SWIGLU>
+int launch_ring(GemmArgs a, hipStream_t st) {
   a.tiles_m = (int)(((int64_t)a.M + BM - 1) / BM);
-  a.tiles_n = (int)(((int64_t)a.N + BN - 1) / BN);
-  const unsigned tiles = (unsigned)a.tiles_m * (unsigned)a.tiles_n;
-  if constexpr (BM == 64 && BN == 64 && WN == 2 && NW == 4) {  // split-K runs 64 x 64 tiles
-    if (a.splits > 1) {
-      if (launch_split_partials(a, st) != EGPT_OK) return EGPT_ERR_LAUNCH;
-      const int64_t mn = (int64_t)a.M * a.N;
-      const unsigned blocks = (unsigned)std::min<int64_t>((mn + kReduceThreads - 1) / kReduceThreads, 4096);
-      if (!launch_reduce<kMaxSplits>(a, blocks, st)) return EGPT_ERR_INVALID;
-      return EGPT_LAUNCH_STATUS();
-    }
-  }
-  if constexpr (BM == 64 && BN == 64 && WN == 2 && NW == 4) {
-    // Fewer tiles than CUs: each block's chain of dependent K steps is the time,
-    // and a 128-wide step halves it (measured on the MI355X: 200 x 2048 -> 2048
-    // 16.5 -> 12.5 us, 160 x 2048 -> 4096 16.8 -> 13.2; with 320 tiles, 300 x 2048
-    // -> 4096, 1.7% slower).
-    if (a.K % kBKSplit == 0 && tiles < 256) {
-      hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, false, 2, 4>), dim3(tiles),
-                         dim3(4 * kWave), 0, st, a);
-      return EGPT_LAUNCH_STATUS();
-    }
-  }
-  hipLaunchKernelGGL((int8_gemm_kernel<BM, BN, kBK, false, WN, NW>), dim3(tiles),
-                     dim3(NW * kWave), 0, st, a);
+  a.tiles_n = SWIGLU ? (int)(((int64_t)a.inter + BN / 2 - 1) / (BN / 2)) : (int)(((int64_t)a.N + BN - 1) / BN);
+  const unsigned blocks = (unsigned)a.tiles_m * (unsigned)a.tiles_n * (unsigned)(SPLIT ? a.splits : 1);
+  hipLaunchKernelGGL((int8_gemm_ring_kernel<BM, BN, WM, WN, STAGES, SPLIT, SWIGLU>), dim3(blocks),
+                     dim3(WM * WN * kWave), 0, st, a);
   return EGPT_LAUNCH_STATUS();
 }
 
-// The LDS-direct tiles (K a multiple of 64); with SWIGLU each block covers 32 TN features.
+// The split slices' fp32 tiles into a.part (a.splits > 1); no reduce.
+int launch_split_partials(const GemmArgs& a, hipStream_t st) {
+  if (a.M <= 32) return launch_ring<32, 64, 1, 4, 3, true, false>(a, st);
+  return launch_ring<64, 64, 2, 4, 3, true, false>(a, st);
+}
+
+int launch_split(const GemmArgs& a, hipStream_t st) {
+  if (launch_split_partials(a, st) != EGPT_OK) return EGPT_ERR_LAUNCH;
+  const int64_t mn = (int64_t)a.M * a.N;
+  const unsigned blocks = (unsigned)std::min<int64_t>((mn + kReduceThreads - 1) / kReduceThreads, 4096);
+  if (!launch_reduce<kMaxSplits>(a, blocks, st)) return EGPT_ERR_INVALID;
+  return EGPT_LAUNCH_STATUS();
+}
+
+// The LDS-direct large tiles; with SWIGLU each block covers 32 TN features.
 template <int TM, int TN, bool SWIGLU>
-int launch_gemm_dma(GemmArgs a, hipStream_t st) {
+int launch_dma(GemmArgs a, hipStream_t st) {
   constexpr int BM = 32 * TM, BN = 64 * TN;
   a.tiles_m = (int)(((int64_t)a.M + BM - 1) / BM);
   a.tiles_n = SWIGLU ? (int)(((int64_t)a.inter + BN / 2 - 1) / (BN / 2)) : (int)(((int64_t)a.N + BN - 1) / BN);
@@ -658,49 +598,48 @@ int launch_gemm_dma(GemmArgs a, hipStream_t st) {
   return EGPT_LAUNCH_STATUS();
 }
 
-// Which LDS-direct tile: the least time of the launch's rounds of 256 blocks (one per CU; the 128 x 128 tile fits two
-// blocks on a CU, and a pair of them takes less than two rounds). The costs are the us of one full round over
-// K = 4096, launch excluded, measured on the MI355X; their ratios hold for other K.
-struct DmaTile {
-  int tm, tn;
+// Which tile: the least time of the launch's rounds of 256 blocks (one per CU; where two blocks fit on a CU, a pair of
+// them takes less than two rounds). The costs are the us of one full round over K = 4096, launch excluded, measured on
+// the MI355X; their ratios hold for other K.
+struct GemmTile {
+  int bm, bn;
   float round;  // 256 blocks
   float pair;   // 512 blocks, where two fit on a CU
+  bool swiglu;  // has the SwiGLU form
+  int (*launch)(GemmArgs, hipStream_t);
+  int (*launch_swiglu)(GemmArgs, hipStream_t);
 };
-constexpr DmaTile kDmaTiles[] = {{8, 4, 95.0f, 0.f}, {6, 4, 79.5f, 0.f}, {8, 3, 79.5f, 0.f}, {6, 3, 65.3f, 0.f},
-                                 {4, 4, 61.7f, 0.f}, {8, 2, 59.5f, 0.f}, {4, 3, 53.8f, 0.f}, {6, 2, 50.0f, 0.f},
-                                 {4, 2, 39.7f, 64.0f}};
+template <int TM, int TN>
+constexpr GemmTile dma_tile(float round, float pair = 0.f) {
+  if constexpr (TN % 2 == 0)
+    return {32 * TM, 64 * TN, round, pair, true, launch_dma<TM, TN, false>, launch_dma<TM, TN, true>};
+  else
+    return {32 * TM, 64 * TN, round, pair, false, launch_dma<TM, TN, false>, nullptr};
+}
+template <int BM, int BN, int WM, int WN, int STAGES>
+constexpr GemmTile ring_tile(float round, float pair = 0.f) {
+  return {BM, BN, round, pair, true, launch_ring<BM, BN, WM, WN, STAGES, false, false>,
+          launch_ring<BM, BN, WM, WN, STAGES, false, true>};
+}
+constexpr GemmTile kGemmTiles[] = {
+    dma_tile<8, 4>(95.0f), dma_tile<6, 4>(79.5f), dma_tile<8, 3>(79.5f), dma_tile<6, 3>(65.3f), dma_tile<4, 4>(61.7f),
+    dma_tile<8, 2>(59.5f), dma_tile<4, 3>(53.8f), dma_tile<6, 2>(50.0f), dma_tile<4, 2>(39.7f, 64.0f),
+    ring_tile<64, 128, 2, 4, 4>(26.5f), ring_tile<128, 64, 2, 4, 3>(23.6f), ring_tile<96, 64, 2, 4, 3>(21.3f),
+    ring_tile<64, 64, 2, 4, 3>(17.3f, 27.0f), ring_tile<32, 64, 1, 4, 3>(14.0f, 24.0f)};
 
-float dma_cost(const DmaTile& t, int64_t M, int64_t N) {
-  const int64_t tiles = ((M + 32 * t.tm - 1) / (32 * t.tm)) * ((N + 64 * t.tn - 1) / (64 * t.tn));
+float tile_cost(const GemmTile& t, int64_t M, int64_t N) {
+  const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
   if (t.pair == 0.f) return t.round * (float)((tiles + 255) / 256);
   const int64_t rest = tiles % 512;
   return t.pair * (float)(tiles / 512) + (rest == 0 ? 0.f : rest <= 256 ? t.round : t.pair);
 }
 
-// N counts a SwiGLU product's gate and up columns; its tiles need an even TN.
-template <bool SWIGLU>
-int launch_gemm_dma_best(const GemmArgs& a, hipStream_t st) {
-  const DmaTile* best = nullptr;
-  for (const DmaTile& t : kDmaTiles)
-    if (!(SWIGLU && t.tn % 2) && (!best || dma_cost(t, a.M, a.N) < dma_cost(*best, a.M, a.N))) best = &t;
-  switch (best->tm * 8 + best->tn) {
-    case 8 * 8 + 4: return launch_gemm_dma<8, 4, SWIGLU>(a, st);
-    case 6 * 8 + 4: return launch_gemm_dma<6, 4, SWIGLU>(a, st);
-    case 4 * 8 + 4: return launch_gemm_dma<4, 4, SWIGLU>(a, st);
-    case 8 * 8 + 2: return launch_gemm_dma<8, 2, SWIGLU>(a, st);
-    case 6 * 8 + 2: return launch_gemm_dma<6, 2, SWIGLU>(a, st);
-    case 4 * 8 + 2: return launch_gemm_dma<4, 2, SWIGLU>(a, st);
-    default: break;
-  }
-  if constexpr (!SWIGLU) {
-    switch (best->tm * 8 + best->tn) {
-      case 8 * 8 + 3: return launch_gemm_dma<8, 3, false>(a, st);
-      case 6 * 8 + 3: return launch_gemm_dma<6, 3, false>(a, st);
-      case 4 * 8 + 3: return launch_gemm_dma<4, 3, false>(a, st);
-      default: break;
-    }
-  }
-  return EGPT_ERR_INVALID;
+// N counts a SwiGLU product's gate and up columns.
+int launch_best_tile(const GemmArgs& a, bool swiglu, hipStream_t st) {
+  const GemmTile* best = nullptr;
+  for (const GemmTile& t : kGemmTiles)
+    if ((t.swiglu || !swiglu) && (!best || tile_cost(t, a.M, a.N) < tile_cost(*best, a.M, a.N))) best = &t;
+  return swiglu ? best->launch_swiglu(a, st) : best->launch(a, st);
 }
 
 // The same product for shapes the MFMA kernel does not take (K not a multiple of
@@ -805,14 +744,10 @@ extern "C" int egpt_int8_gemm_ws(const void* x, int64_t ldx, const int8_t* w, in
       a.splits = splits;
       a.kchunk = kchunk;
       a.part = (float*)workspace;
-      return launch_gemm<64, 64>(a, stream);
+      return launch_split(a, stream);
     }
   }
-  // The LDS-direct tiles from kDmaMinTiles tiles of their smallest size; below, the 64-row tiles, whose more and
-  // shorter blocks fill more of the chip.
-  if (M > 64 && gemm_blocks<128, 128>(a) >= kDmaMinTiles) return launch_gemm_dma_best<false>(a, stream);
-  if (M > 64 && gemm_blocks<128, 64>(a) >= 256) return launch_gemm<128, 64>(a, stream);
-  return launch_gemm<64, 64>(a, stream);
+  return launch_best_tile(a, false, stream);
 }
 
 extern "C" int egpt_int8_gemm_swiglu(const void* x, int64_t ldx, const int8_t* w, int64_t ldw, const float* scale,
@@ -827,23 +762,11 @@ extern "C" int egpt_int8_gemm_swiglu(const void* x, int64_t ldx, const int8_t* w
     return EGPT_ERR_UNSUPPORTED;
   GemmArgs a{(const uint16_t*)x, ldx, w, ldw, scale, (uint16_t*)act, ld_act, M, (int)N, K, 0, 0, 1, K, nullptr,
              inter};
-  // The LDS-direct tiles where the plain product would take them.
-  if (M > 64 && gemm_blocks<128, 128>(a) >= kDmaMinTiles) return launch_gemm_dma_best<true>(a, stream);
-  // 64 x 64 tiles (32 features each, gate and up in the two halves of a wavefront's tile) where the plain
-  // product would run them too: not where it would split K, which this form cannot.
+  // Not where the plain product would split K, which this form cannot.
   int splits, kchunk;
   gemm_split(M, N, K, splits, kchunk);
   if (splits > 1 || N > INT32_MAX / 2) return EGPT_ERR_UNSUPPORTED;
-  a.tiles_m = (M + 63) / 64;
-  a.tiles_n = (inter + 31) / 32;
-  const unsigned tiles = (unsigned)a.tiles_m * (unsigned)a.tiles_n;
-  if (K % kBKSplit == 0 && tiles < 256)
-    hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBKSplit, false, 2, 4, true>), dim3(tiles),
-                       dim3(4 * kWave), 0, stream, a);
-  else
-    hipLaunchKernelGGL((int8_gemm_kernel<64, 64, kBK, false, 2, 4, true>), dim3(tiles),
-                       dim3(4 * kWave), 0, stream, a);
-  return EGPT_LAUNCH_STATUS();
+  return launch_best_tile(a, true, stream);
 }
 
 extern "C" int egpt_int8_gemm_add_rmsnorm(const void* x, int64_t ldx, const int8_t* w, int64_t ldw,

@@ -334,6 +334,38 @@ def test_gemm_swiglu_lds_direct_tiles_match_the_two_calls(tile, m, k, inter):
     assert torch.equal(one, two)
 
 
+# the small tiles (rows x features of a block) and shapes that take each: 1 to 17 steps of 128 K columns through rings of
+# 3 and 4 stages, a last step of 64, ragged rows and features, an odd output pitch
+RING_TILE_SHAPES = [('32x64', 20, 64, 77), ('32x64', 17, 192, 200), ('32x64', 100, 1088, 130), ('64x64', 256, 128, 4090),
+                    ('64x64', 100, 2112, 8000), ('64x64', 190, 320, 5300), ('96x64', 77, 192, 12290),
+                    ('96x64', 96, 576, 12290), ('128x64', 120, 320, 12290), ('128x64', 250, 448, 6150),
+                    ('64x128', 60, 64, 20001), ('64x128', 190, 704, 9000)]
+
+
+@pytest.mark.parametrize('tile,m,k,n', RING_TILE_SHAPES)
+def test_prefill_gemm_small_tiles_match_oracle(tile, m, k, n):
+    """egpt_int8_gemm without a workspace (K is not split) on the small tiles, against the oracle's prefill formula, and
+    with an even feature count egpt_int8_gemm_swiglu against the same product followed by egpt_silu_mul, bit for bit."""
+    from efficientgpt_amd import _lib
+    lib = _lib.lib()
+    x, q, s = make_case(m, k, n, seed=m + k + n)
+    xd, qd, sd = x.cuda(), q.cuda(), s.cuda()
+    y = torch.full((m, n + 3), -7.0, device='cuda', dtype=torch.bfloat16)
+    assert lib.egpt_int8_gemm(xd.data_ptr(), k, qd.data_ptr(), k, sd.data_ptr(), y.data_ptr(), n + 3, m, n, k,
+                              _lib.stream_ptr()) == 0
+    check_against_oracle(y[:, :n].cpu(), x, q, s)
+    assert bool((y[:, n:] == -7).all())
+    if n % 2 or k % 128 == 0:
+        return
+    inter = n // 2
+    gu = y[:, :n].contiguous()
+    two, one = (torch.full((m, inter), -7.0, device='cuda', dtype=torch.bfloat16) for _ in range(2))
+    assert lib.egpt_silu_mul(gu.data_ptr(), n, inter, two.data_ptr(), inter, m, _lib.stream_ptr()) == 0
+    assert lib.egpt_int8_gemm_swiglu(xd.data_ptr(), k, qd.data_ptr(), k, sd.data_ptr(), one.data_ptr(), inter, m, inter,
+                                     k, _lib.stream_ptr()) == 0
+    assert torch.equal(one, two)
+
+
 SPLIT_SHAPES = [(128, 6144, 2048), (128, 2048, 4096), (33, 6144, 2048), (64, 2048, 2048), (100, 4096, 1000),
                 (17, 12288, 64), (200, 2048, 2048), (130, 2048, 2000), (256, 2048, 2048)]
 
