@@ -75,6 +75,8 @@ SIGNATURES = {
     'egpt_argmax': (_c_int, [_c_vp, _c_int, _c_vp, _c_size, _c_vp, _c_vp, _c_vp]),
     'egpt_qwen3_step_workspace': (_c_int, [_c_vp, ctypes.POINTER(_c_size)]),
     'egpt_qwen3_decode_step': (_c_int, [_c_vp, _c_vp]),
+    'egpt_qwen3_prefill_workspace': (_c_int, [_c_vp, _c_int, ctypes.POINTER(_c_size)]),
+    'egpt_qwen3_prefill': (_c_int, [_c_vp, _c_vp, _c_int, _c_int, _c_int, _c_vp, _c_size, _c_vp]),
     'egpt_qwen3_step_gemvs': (_c_int, [_c_vp, _c_vp, _c_int, ctypes.POINTER(_c_int)]),
     'egpt_int8_gemv_fused_parts': (_c_int, [_c_vp, ctypes.POINTER(_c_int)]),
     'egpt_int8_gemv_fused': (_c_int, [_c_vp, _c_vp]),

@@ -566,6 +566,16 @@ class Qwen3Int8Engine:
             raise ValueError('prefill needs at least one token')
         if pos0 + t > self.cap:
             raise ValueError('prompt exceeds the cache capacity')
+        lib = _lib.lib()
+        if self.fold_norms:
+            need = ctypes.c_size_t()
+            _lib.check('egpt_qwen3_prefill_workspace', lib.egpt_qwen3_prefill_workspace(ctypes.byref(self._step_c), t,
+                                                                                        ctypes.byref(need)))
+            ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
+            _lib.check('egpt_qwen3_prefill', lib.egpt_qwen3_prefill(
+                ctypes.byref(self._step_c), ids.data_ptr(), t, pos0, int(use_prompt_kernel(t, pos0)), ws.data_ptr(),
+                need.value, self._stream()))
+            return self.logits[0]
         positions = torch.arange(pos0, pos0 + t, device=dev, dtype=torch.long)
         x = torch.empty(t, c.hidden, device=dev, dtype=bf)
         h = torch.empty_like(x)
@@ -576,7 +586,6 @@ class Qwen3Int8Engine:
         gu = torch.empty(t, 2 * c.inter, device=dev, dtype=bf)
         act = torch.empty(t, c.inter, device=dev, dtype=bf)
         down = torch.empty_like(x)
-        lib = _lib.lib()
         _lib.check('egpt_embed', lib.egpt_embed(ids.data_ptr(), t, self.embed.data_ptr(), self.embed.stride(0),
                                                 c.vocab, x.data_ptr(), x.stride(0), c.hidden, self._stream()))
         ws = self._prefill_workspace(t) if t > MAX_DECODE_ROWS else None

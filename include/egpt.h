@@ -86,7 +86,7 @@ int egpt_quantize_rows(int dtype, const void *w, int64_t ldw, int N, int K, int8
  * without materialising the bf16 weights. x bf16 [M, K] (row stride ldx), w int8 [N, K]
  * (ldw), y bf16 [M, N] (ldy). The MFMA kernel takes K a multiple of 64, ldx % 8 == 0,
  * ldw % 16 == 0, 16-byte aligned x and w and operands under 2 GiB; any other shape runs
- * a generic kernel (fp32 sums over lane-strided K, the same two roundings), slower but
+ * a kernel of 64 x 64 MFMA tiles with loads of any alignment, slower but
  * with the same contract.
  */
 int egpt_int8_gemm(const void *x, int64_t ldx, const int8_t *w, int64_t ldw, const float *scale,
@@ -402,6 +402,17 @@ int egpt_qwen3_step_workspace(const egpt_qwen3_step *step, size_t *bytes);
  * SDPA. */
 int egpt_qwen3_step_default_splits(int heads, int kv_heads, int head_dim, int cap);
 int egpt_qwen3_decode_step(const egpt_qwen3_step *step, hipStream_t stream);
+
+/* The prompt pass: `rows` token ids (device memory) at positions pos0 .. pos0 + rows - 1 through the model of
+ * `step`, reading its weights, RoPE tables and caches. Writes K/V slots pos0 .. pos0 + rows - 1 of every layer, the
+ * last row's logits and their greedy pick into *token, and sets *position to pos0 + rows. Every linear is the int8
+ * linear's formula for `rows` rows (at most EGPT_MAX_DECODE_ROWS: the GEMV; more: the prefill GEMM,
+ * research/realmodel/int8_linear.py:88-97). prompt_attn: attention by egpt_prefill_attn, else by egpt_decode_attn with
+ * the prompt rows as batch rows. The workspace (egpt_qwen3_prefill_workspace bytes, 256-byte aligned) holds the pass's
+ * activations; its contents on entry do not matter. hidden <= 16384. */
+int egpt_qwen3_prefill_workspace(const egpt_qwen3_step *step, int rows, size_t *bytes);
+int egpt_qwen3_prefill(const egpt_qwen3_step *step, const int64_t *tokens, int rows, int pos0, int prompt_attn,
+                       void *workspace, size_t workspace_bytes, hipStream_t stream);
 
 /* The step's fused GEMV launches as egpt_gemv_fused descriptions, in launch
  * order (4 per layer, then the head): *count = 4 layers + 1; `out` (capacity

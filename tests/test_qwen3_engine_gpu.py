@@ -143,6 +143,30 @@ def test_fused_step_matches_unfused_step(shape, std, cap, plen):
     assert agree >= 11, (tu, tf)
 
 
+@pytest.mark.parametrize('plen,pos0', [(1, 0), (1, 30), (2, 9), (5, 0), (16, 0), (17, 3), (65, 90), (66, 120), (300, 11)])
+def test_prefill_one_call_equals_separate_calls(plen, pos0):
+    """egpt_qwen3_prefill (every launch of the pass from one call; embedding, first norm and positions in one kernel) at
+    the edges of its row rules (one row, the decode GEMV's 16, the prompt attention's 64 rows and 160 positions), from
+    an empty and a filled cache, against one call per op from Python: logits, caches, token and position bit for bit.
+    Token ids out of the vocabulary are clamped alike."""
+    eng, _ = build(SMALL, seed=13, std=0.15, cap=512)
+    gen = torch.Generator().manual_seed(plen + pos0)
+    prompt = torch.randint(0, SMALL.vocab, (plen,), generator=gen)
+    prompt[plen // 2] = SMALL.vocab + 5
+    before = torch.randn(eng.k_cache[:, :, :max(pos0, 1)].shape, generator=gen).to(torch.bfloat16).cuda()
+    out = []
+    for fold in (True, False):
+        eng.fold_norms = fold
+        eng.reset()
+        eng.k_cache[:, :, :pos0] = before[:, :, :pos0]
+        eng.v_cache[:, :, :pos0] = before[:, :, :pos0] * 0.5
+        logits = eng.prefill(prompt, pos0).clone()
+        out.append((logits, eng.k_cache.clone(), eng.v_cache.clone(), int(eng.token), int(eng.position)))
+    (la, ka, va, ta, pa), (lb, kb, vb, tb, pb) = out
+    assert torch.equal(la, lb) and torch.equal(ka, kb) and torch.equal(va, vb)
+    assert (ta, pa) == (tb, pb) and pa == pos0 + plen
+
+
 @pytest.mark.parametrize('shape', [SMALL, SMALL8])
 @pytest.mark.parametrize('plen', [40, 128, 4096])
 def test_prefill_folded_norms_equal_separate_calls(shape, plen):
