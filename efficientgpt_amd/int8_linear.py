@@ -101,8 +101,8 @@ def int8_gemm(x2, w, s, out=None, workspace=None):
     directly (no bf16 copy of them). Measured on the MI355X against the reference's dequantise-then-library-GEMM
     formula at the Qwen3-1.7B and Qwen3-8B shapes: 1.2-2.9x faster at 128 rows, 1.1-1.4x at 1024-2048, and at
     8192 rows 0.93-1.4x (faster on 14 of 16 shapes, the whole 8B layer 8% faster). Shapes the MFMA kernel does
-    not take (K not a multiple of 64, unaligned rows, operands of 2 GiB or more) run the library's generic kernel,
-    the same formula without MFMA."""
+    not take (K not a multiple of 64, unaligned rows, operands of 2 GiB or more) run the library's ragged kernel,
+    the same formula on smaller tiles with loads of any alignment."""
     m, k = x2.shape
     n = w.shape[0]
     if x2.stride(1) != 1:

@@ -424,6 +424,28 @@ def test_prefill_generic_kernel_for_shapes_the_mfma_kernel_refuses(m, k, n):
     assert torch.equal(int8_linear(xd, qd, sd), y)  # the op takes the same kernel
 
 
+@pytest.mark.parametrize('m', [1, 2, 4, 5, 9, 16, 17, 65, 150])
+@pytest.mark.parametrize('k,n', [(1, 5), (7, 70), (16, 65), (65, 130), (127, 3), (193, 64), (1040, 200), (2063, 77)])
+def test_shapes_and_alignments_of_no_kind(m, k, n):
+    """K below, at and past the chunks of the ragged kernels (16 columns a lane, 64 a step, 1024 a wavefront), rows of x
+    and of the weights off every alignment, at the row counts of each GEMV form and of the GEMM's tiles, between values
+    that would show if a load past a row's end were multiplied; against the oracle."""
+    from efficientgpt_amd import _lib
+    lib = _lib.lib()
+    x, q, s = make_case(m, k, n, seed=m + 7 * k + n)
+    xb = torch.full((m, k + 3), float('nan'), dtype=torch.bfloat16)
+    xb[:, 1:k + 1] = x
+    qb = torch.full((n, k + 5), 119, dtype=torch.int8)
+    qb[:, 3:k + 3] = q
+    xd, qd, sd = xb.cuda()[:, 1:k + 1], qb.cuda()[:, 3:k + 3], s.cuda()
+    y = torch.full((m, n + 1), -7.0, device='cuda', dtype=torch.bfloat16)
+    fn = lib.egpt_int8_gemv if m <= 16 else lib.egpt_int8_gemm
+    assert fn(xd.data_ptr(), k + 3, qd.data_ptr(), k + 5, sd.data_ptr(), y.data_ptr(), n + 1, m, n, k,
+              _lib.stream_ptr()) == 0
+    check_against_oracle(y[:, :n].cpu(), x, q, s)
+    assert bool((y[:, n:] == -7).all())
+
+
 def test_prefill_op_keeps_leading_dims():
     from efficientgpt_amd.int8_linear import int8_linear
     x, q, s = make_case(48, 2048, 512, seed=11)
