@@ -892,9 +892,14 @@ int launch_r(const FusedGemv& a, int nch, unsigned blocks, hipStream_t st) {
 }
 
 // Blocks of a fused GEMV launch: one tile per wavefront, except the lm_head,
-// whose grid is capped (about four 8-wave blocks per CU) so each block stages
-// the activation once and reduces its argmax once over many tiles.
-constexpr unsigned kHeadMaxBlocks = 1024;
+// whose grid is capped at two 8-wave blocks per CU, so each block stages and
+// normalises the activation once and reduces its argmax once over many tiles.
+// Measured on the MI355X (us, a decode step of four Qwen3-1.7B / two Qwen3-8B
+// layers, the head 311 / 622 MB of it): 256 blocks 153.6 / 218.6, 384 152.5 / 237,
+// 512 150.8 / 219.5, 640 157.8 / 231.4, 768 154.6 / 222.4, 1024 150.8 / 224.5,
+// 1280 152.0 / 226.5, uncapped 187 / 300. Grids that give every wavefront the same
+// number of tiles were no better (512: 150.3 / 220.9).
+constexpr unsigned kHeadMaxBlocks = 512;
 
 unsigned gemv_blocks(int64_t n, bool pairs, bool capped) {
   const int rh = features_per_wave(n, pairs);
