@@ -23,7 +23,7 @@ Step (token t at position p; writes K/V slot p, attends to slots 0..p):
   embed -> [add+]RMSNorm -> QKV GEMV -> q/k norm + RoPE + cache write -> split-K
   attention + combine -> o GEMV -> add+RMSNorm -> gate_up GEMV -> SiLU*up ->
   down GEMV -> ... -> add+final RMSNorm -> lm_head GEMV -> argmax (token, p + 1).
-Prefill runs the same kernels over all prompt rows, outside the graph; linears past 16
+Prefill (egpt_qwen3_prefill) runs all prompt rows through the model from one call, outside the graph; linears past 16
 rows take the reference's prefill formula (int8_linear.py:96-97) on the MFMA GEMM that
 reads the int8 weights, and long prompts (use_prompt_kernel) the causal MFMA prefill
 attention (egpt_prefill_attn).
@@ -209,11 +209,10 @@ class Qwen3Int8Engine:
         def put(t, dtype=None):
             return t.to(device=dev, dtype=dtype or t.dtype).contiguous()
 
-        # Prompt passes fold the residual add + RMSNorm after o_proj and down_proj into the split-K GEMM's reduce
-        # (egpt_int8_gemm_add_rmsnorm), q/k norm + RoPE into the split-K QKV reduce (egpt_int8_gemm_qk_norm_rope),
-        # the next layer's input norm into the down projection and SwiGLU into the gate/up GEMM
-        # (egpt_int8_gemm_swiglu); False runs the separate linear, egpt_add_rmsnorm, egpt_qk_norm_rope and
-        # egpt_silu_mul calls instead (the same bits).
+        # Prompt passes run from one call (egpt_qwen3_prefill), which folds the residual add + RMSNorm after o_proj and
+        # down_proj into the split-K GEMM's reduce, q/k norm + RoPE into the split-K QKV reduce and SwiGLU into the
+        # gate/up GEMM; False runs a call per op instead: egpt_embed, the norms, the linears, egpt_qk_norm_rope,
+        # egpt_silu_mul (the same bits).
         self.fold_norms = True
         pk = weights if packed else pack_qwen3(c, weights)
         check_packed(c, pk)
@@ -389,9 +388,9 @@ class Qwen3Int8Engine:
         return _lib.stream_ptr(self.device)
 
     def _prefill_workspace(self, rows):
-        """One split-K workspace for a prompt pass of `rows` rows: the largest any of the layer's linears (and
-        their fused reduce) needs at that row count, allocated once per pass and shared by every GEMM of it
-        (the calls run in stream order, so none overlaps another)."""
+        """One split-K workspace for a prompt pass of `rows` rows: the largest any of the layer's linears needs at that
+        row count, allocated once per pass and shared by every GEMM of it (the calls run in stream order, so none
+        overlaps another)."""
         lib, c = _lib.lib(), self.cfg
         d = c.head_dim
         need, most = ctypes.c_size_t(), 0
@@ -411,41 +410,19 @@ class Qwen3Int8Engine:
             int8_gemm(x[:rows], q, s, out=out[:rows], workspace=ws)
 
     def _linear_add_norm(self, xin, q, s, out, x, norm_w, h, rows, ws=None):
-        """x = bf16(x + linear(xin)) and h = RMSNorm(x) * norm_w for `rows` rows. Split-K shapes take
-        egpt_int8_gemm_add_rmsnorm (one launch after the split slices instead of the reduce and the norm, the
-        same bits); the others, or every shape when `fold_norms` is off, the linear into `out`, then
-        egpt_add_rmsnorm."""
+        """x = bf16(x + linear(xin)) and h = RMSNorm(x) * norm_w for `rows` rows."""
         lib, c, st = _lib.lib(), self.cfg, self._stream()
-        if rows > MAX_DECODE_ROWS and self.fold_norms:
-            need = ctypes.c_size_t()
-            _lib.check('egpt_int8_gemm_workspace',
-                       lib.egpt_int8_gemm_workspace(rows, q.shape[0], q.shape[1], ctypes.byref(need)))
-            if need.value:
-                if ws is None or ws.numel() < need.value:
-                    ws = torch.empty(need.value, device=self.device, dtype=torch.uint8)
-                r = lib.egpt_int8_gemm_add_rmsnorm(xin.data_ptr(), xin.stride(0), q.data_ptr(), q.stride(0),
-                                                   s.data_ptr(), x.data_ptr(), x.stride(0), norm_w.data_ptr(),
-                                                   h.data_ptr(), h.stride(0), rows, q.shape[0], q.shape[1], c.rms_eps,
-                                                   ws.data_ptr(), ws.numel(), st)
-                if r != _lib.EGPT_ERR_UNSUPPORTED:
-                    _lib.check('egpt_int8_gemm_add_rmsnorm', r)
-                    return
         self._linear(xin, q, s, out, rows, ws)
         _lib.check('egpt_add_rmsnorm', lib.egpt_add_rmsnorm(x.data_ptr(), x.stride(0), out.data_ptr(), out.stride(0),
                                                             norm_w.data_ptr(), h.data_ptr(), h.stride(0), rows,
                                                             c.hidden, c.rms_eps, st))
 
-    def _layer(self, i, rows, x, h, qkv, qrot, attn, o, gu, act, down, positions, pos_stride, first, pos0=0,
-               normed=False, ws=None):
-        """One layer over `rows` rows. `normed`: h already holds the layer's input RMSNorm (the previous layer's
-        down projection folded it in); the layer then folds the next layer's input norm into its own down
-        projection when there is a next layer (returns True), and leaves x + down to the caller otherwise. `ws`:
-        the pass's split-K workspace (_prefill_workspace)."""
+    def _layer(self, i, rows, x, h, qkv, qrot, attn, o, gu, act, down, positions, pos_stride, first, pos0=0, ws=None):
+        """One layer over `rows` rows, one call per op; leaves x + down to the next layer or the head. `ws`: the
+        pass's split-K workspace (_prefill_workspace)."""
         lib, c, L, st = _lib.lib(), self.cfg, self.layers[i], self._stream()
         d = c.head_dim
-        if normed:
-            pass
-        elif first:
+        if first:
             _lib.check('egpt_rmsnorm', lib.egpt_rmsnorm(x.data_ptr(), x.stride(0), L['in_w'].data_ptr(), h.data_ptr(),
                                                         h.stride(0), rows, c.hidden, c.rms_eps, st))
         else:
@@ -453,23 +430,11 @@ class Qwen3Int8Engine:
                 x.data_ptr(), x.stride(0), down.data_ptr(), down.stride(0), L['in_w'].data_ptr(), h.data_ptr(),
                 h.stride(0), rows, c.hidden, c.rms_eps, st))
         kc, vc = self.k_cache[i], self.v_cache[i]
-        fused = _lib.EGPT_ERR_UNSUPPORTED
-        if rows > MAX_DECODE_ROWS and self.fold_norms and ws is not None:
-            # split-K QKV: the reduce, q/k norm, RoPE and cache write in one launch after the split slices
-            fused = lib.egpt_int8_gemm_qk_norm_rope(
-                h.data_ptr(), h.stride(0), L['qkv_q'].data_ptr(), L['qkv_q'].stride(0), L['qkv_s'].data_ptr(),
-                positions.data_ptr(), L['qn_w'].data_ptr(), L['kn_w'].data_ptr(), self.cos.data_ptr(),
-                self.sin.data_ptr(), qrot.data_ptr(), qrot.stride(0), kc.data_ptr(), vc.data_ptr(), kc.stride(0),
-                kc.stride(1), rows, c.heads, c.kv_heads, d, c.hidden, self.cap, c.rms_eps, ws.data_ptr(), ws.numel(),
-                st)
-        if fused == _lib.EGPT_ERR_UNSUPPORTED:
-            self._linear(h, L['qkv_q'], L['qkv_s'], qkv, rows, ws)
-            _lib.check('egpt_qk_norm_rope', lib.egpt_qk_norm_rope(
-                qkv.data_ptr(), qkv.stride(0), positions.data_ptr(), L['qn_w'].data_ptr(), L['kn_w'].data_ptr(),
-                self.cos.data_ptr(), self.sin.data_ptr(), qrot.data_ptr(), qrot.stride(0), kc.data_ptr(),
-                vc.data_ptr(), kc.stride(0), kc.stride(1), rows, c.heads, c.kv_heads, d, self.cap, c.rms_eps, st))
-        else:
-            _lib.check('egpt_int8_gemm_qk_norm_rope', fused)
+        self._linear(h, L['qkv_q'], L['qkv_s'], qkv, rows, ws)
+        _lib.check('egpt_qk_norm_rope', lib.egpt_qk_norm_rope(
+            qkv.data_ptr(), qkv.stride(0), positions.data_ptr(), L['qn_w'].data_ptr(), L['kn_w'].data_ptr(),
+            self.cos.data_ptr(), self.sin.data_ptr(), qrot.data_ptr(), qrot.stride(0), kc.data_ptr(),
+            vc.data_ptr(), kc.stride(0), kc.stride(1), rows, c.heads, c.kv_heads, d, self.cap, c.rms_eps, st))
         if use_prompt_kernel(rows, pos0):
             _lib.check('egpt_prefill_attn', lib.egpt_prefill_attn(
                 qrot.data_ptr(), qrot.stride(0), kc.data_ptr(), vc.data_ptr(), kc.stride(0), kc.stride(1),
@@ -477,23 +442,10 @@ class Qwen3Int8Engine:
         else:
             self._kernel_attention(qrot, kc, vc, rows, positions, pos_stride, attn)
         self._linear_add_norm(attn, L['o_q'], L['o_s'], o, x, L['post_w'], h, rows, ws)
-        fused = _lib.EGPT_ERR_UNSUPPORTED
-        if rows > MAX_DECODE_ROWS and self.fold_norms:  # SwiGLU in the gate/up GEMM's epilogue
-            fused = lib.egpt_int8_gemm_swiglu(h.data_ptr(), h.stride(0), L['gu_q'].data_ptr(), L['gu_q'].stride(0),
-                                              L['gu_s'].data_ptr(), act.data_ptr(), act.stride(0), rows, c.inter,
-                                              c.hidden, st)
-        if fused == _lib.EGPT_ERR_UNSUPPORTED:
-            self._linear(h, L['gu_q'], L['gu_s'], gu, rows, ws)
-            _lib.check('egpt_silu_mul', lib.egpt_silu_mul(gu.data_ptr(), gu.stride(0), c.inter, act.data_ptr(),
-                                                          act.stride(0), rows, st))
-        else:
-            _lib.check('egpt_int8_gemm_swiglu', fused)
-        if i + 1 < c.layers and rows > MAX_DECODE_ROWS and self.fold_norms:
-            # the next layer's input norm folds into this projection
-            self._linear_add_norm(act, L['down_q'], L['down_s'], down, x, self.layers[i + 1]['in_w'], h, rows, ws)
-            return True
+        self._linear(h, L['gu_q'], L['gu_s'], gu, rows, ws)
+        _lib.check('egpt_silu_mul', lib.egpt_silu_mul(gu.data_ptr(), gu.stride(0), c.inter, act.data_ptr(),
+                                                      act.stride(0), rows, st))
         self._linear(act, L['down_q'], L['down_s'], down, rows, ws)
-        return False
 
     def _kernel_attention(self, qrot, kc, vc, rows, positions, pos_stride, attn):
         """Split-K attention of `rows` query rows over the shared cache (each row a batch row, batch stride 0)."""
@@ -589,10 +541,8 @@ class Qwen3Int8Engine:
         _lib.check('egpt_embed', lib.egpt_embed(ids.data_ptr(), t, self.embed.data_ptr(), self.embed.stride(0),
                                                 c.vocab, x.data_ptr(), x.stride(0), c.hidden, self._stream()))
         ws = self._prefill_workspace(t) if t > MAX_DECODE_ROWS else None
-        normed = False
         for i in range(c.layers):
-            normed = self._layer(i, t, x, h, qkv, qrot, attn, o, gu, act, down, positions, 1, first=(i == 0),
-                                 pos0=pos0, normed=normed, ws=ws)
+            self._layer(i, t, x, h, qkv, qrot, attn, o, gu, act, down, positions, 1, first=(i == 0), pos0=pos0, ws=ws)
         self.position.fill_(pos0 + t - 1)  # argmax advances it to pos0 + t
         self._head(x[t - 1:], down[t - 1:], h[t - 1:])
         return self.logits[0]
