@@ -52,6 +52,9 @@ constexpr int kPfThreads = kPfWaves * 64;
 constexpr float kPfLog2e = 1.4426950408889634f;
 constexpr float kPfLazy = 8.f;  // exponent by which a score may pass the softmax's reference maximum (p < 2^8)
 
+// Blocks up to which a prompt takes the two-group form: its blocks, twice as many, still fit the 256 CUs in one round.
+constexpr int kPfSmallGrid = 128;
+
 struct PrefillArgs {
   const uint16_t* q;
   int64_t q_ld;
@@ -77,7 +80,15 @@ __device__ __forceinline__ uint2 lds_read_tr16(const char* p) {
 }
 
 // D: head dim (32, 64 or 128), a multiple of the MFMA's 32 output rows.
-template <int D>
+//
+// KVG 2, for prompts whose blocks would leave half the CUs idle: wavefronts w and w + 4 share 32 query rows and take the
+// even and the odd tiles (a pair of tiles staged at a time, two pairs in LDS), so a block covers half the rows and twice
+// as many blocks walk half as many tiles each; the two states are merged through LDS at the end. What bounds such a
+// prompt is each wavefront's chain over its tiles, 1.8 us a tile, whether one wavefront or two run on a SIMD (blocks of
+// four wavefronts over half the rows were only 0-15% faster). Measured on the MI355X, one group -> two, us, 16 / 8 heads,
+// D 128: 128 rows over 1000 slots 37.0 -> 24.3, 300 over 2000 65.8 -> 41.5, 600 rows 22.9 -> 16.8, 600 over 1000 47.0 ->
+// 32.4, 2048 rows 60.7 -> 39.1; 32 / 8 heads 1024 rows 34.5 -> 24.2; a prompt of 65 rows over 96 10.6 -> 11.1, the merge.
+template <int D, int KVG>
 __global__ __launch_bounds__(kPfThreads, 1) void prefill_attn_kernel(const PrefillArgs a) {
   constexpr int kPfD = D;
   constexpr int kChunks = kPfD / 8;     // 16-byte chunks per K/V row (slot)
@@ -90,7 +101,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attn_kernel(const Prefi
   // so the four rows x 64 bytes of a transposing read pass do.
   auto kswz = [](int r) { return (r >> (4 - kLogC)) & (kChunks - 1); };
   auto vswz = [](int r) { return 4 * ((r & 3) >> (4 - kLogC)); };
-  __shared__ __align__(16) char Ks[3][kTile];
+  __shared__ __align__(16) char Ks[KVG == 2 ? 4 : 3][kTile];
   __shared__ __align__(16) char Vs[4][kTile];
 
   const int tid = threadIdx.x;
@@ -107,8 +118,9 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attn_kernel(const Prefi
   const int ptile = a.ntiles - 1 - (int)blockIdx.y;
   const int t0 = ptile * a.bt;
   const int wph = a.bt / 32;  // wavefronts per query head
-  const int hq = hk * a.group + sub * a.hb + wave / wph;
-  const int tw = t0 + (wave % wph) * 32;  // the wavefront's first query row
+  const int qw = wave % (kPfWaves / KVG), grp = wave / (kPfWaves / KVG);
+  const int hq = hk * a.group + sub * a.hb + qw / wph;
+  const int tw = t0 + (qw % wph) * 32;    // the wavefront's first query row
   const int tq = tw + col;                // this lane's query row
   const int64_t qpos = (int64_t)a.pos0 + tq;
   // Slots this block visits: 0 .. its last query's position.
@@ -136,10 +148,28 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attn_kernel(const Prefi
     }
   };
 
+  // KVG 2: the tiles 2 jj and 2 jj + 1, K then V, into half jj % 2 of the buffers.
+  auto issue_pair = [&](int jj) {
+#pragma unroll
+    for (int q = 0; q < 2 * kTileLoads; ++q) {
+      const int t = wave + kPfWaves * q;
+      const bool isk = t < 2 * kTile / 1024;  // wave-uniform
+      const int blk = isk ? t : t - 2 * kTile / 1024;
+      const int row = blk * (1024 / kRow) + lane / kChunks;  // of the pair's 2 * kPfSlots
+      const int c = (lane % kChunks) ^ (isk ? kswz(row % kPfSlots) : vswz(row % kPfSlots));
+      const int64_t sl = min((int64_t)jj * 2 * kPfSlots + row, last);
+      lds_load16((isk ? kbase : vbase) + (uint32_t)((jj % 2) * 2 * kTile + blk * 1024),
+                 (isk ? kb : vb) + sl * a.c_sn + 8 * c);
+    }
+  };
+
   // B fragments of Q^T: this lane's query, dims 16 kk + 8 half .. + 7, loaded while tile 0 is, and waited for
   // before the loop: the compiler does not see the LDS-direct loads, so a load of its own still pending in the
   // loop would make it wait for every load in flight before each q . k.
-  issue(0);
+  if constexpr (KVG == 2)
+    issue_pair(0);
+  else
+    issue(0);
   u32x4 qf[kPfD / 16];
   {
     const uint16_t* qrow = a.q + (int64_t)min(tq, a.rows - 1) * a.q_ld + (int64_t)hq * kPfD + 8 * half;
@@ -147,7 +177,7 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attn_kernel(const Prefi
     for (int kk = 0; kk < kPfD / 16; ++kk) qf[kk] = ld16(qrow + 16 * kk);
   }
   EGPT_WAIT_VMCNT(0);
-  if (nt > 1) issue(1);
+  if (KVG == 1 && nt > 1) issue(1);
 
   f32x16_pf o[kPfD / 32];
 #pragma unroll
@@ -253,47 +283,92 @@ __global__ __launch_bounds__(kPfThreads, 1) void prefill_attn_kernel(const Prefi
     }
   };
 
-  // Wavefronts 4-7 run a phase behind 0-3: in the iteration of tile j they
-  // multiply tile j - 1's p . v first, then tile j's q . k and softmax, so while
-  // the wavefront beside them on their SIMD is in its softmax (VALU) they are in
-  // q . k, and in their softmax it is in p . v (MFMA). V tiles stay for one more
-  // iteration, so V rotates through four LDS buffers and K through three. Every
-  // output accumulator takes the same operations in the same order either way.
-  const bool lag = wave >= kPfWaves / 2;  // wave-uniform
-  u32x4 pprev[4];
-  // Tile j: wait for this wavefront's loads of tile j (tile j + 1's stay in flight), publish them with the
-  // barrier, which also retires every wavefront's reads of K tile j - 1 and V tile j - 2, load tile j + 2 into
-  // those buffers, multiply tile j.
+  if constexpr (KVG == 2) {
+    const int np = (nt + 1) / 2;
 #pragma unroll 1
-  for (int j = 0; j < nt; ++j) {
-    if (j + 1 < nt)
-      EGPT_WAIT_VMCNT(kTileLoads);
-    else
+    for (int jj = 0; jj < np; ++jj) {
       EGPT_WAIT_VMCNT(0);
-    lds_barrier();
-    if (j + 2 < nt) issue(j + 2);
-    const int kbuf = j % 3, vbuf = j % 4;
-    f32x16_pf st[2];
-    // A wavefront raises its issue priority for its MFMA phases, so that where both wavefronts of a SIMD are
-    // ready the one feeding the matrix core goes first and the other's softmax fills in behind it.
-    if (!lag) {
-      u32x4 pb[4];
-      __builtin_amdgcn_s_setprio(1);
-      qk(kbuf, st);
-      __builtin_amdgcn_s_setprio(0);
-      softmax(j, st, pb);
-      __builtin_amdgcn_s_setprio(1);
-      pv(vbuf, pb);
-      __builtin_amdgcn_s_setprio(0);
-    } else {
-      __builtin_amdgcn_s_setprio(1);
-      if (j > 0) pv(vbuf == 0 ? 3 : vbuf - 1, pprev);
-      qk(kbuf, st);
-      __builtin_amdgcn_s_setprio(0);
-      softmax(j, st, pprev);
+      lds_barrier();  // publishes pair jj; every wavefront has read pair jj - 1, whose buffers take the next
+      if (jj + 1 < np) issue_pair(jj + 1);
+      const int j = 2 * jj + grp, buf = (jj % 2) * 2 + grp;
+      if (j < nt) {
+        f32x16_pf st[2];
+        u32x4 pb[4];
+        __builtin_amdgcn_s_setprio(1);
+        qk(buf, st);
+        __builtin_amdgcn_s_setprio(0);
+        softmax(j, st, pb);
+        __builtin_amdgcn_s_setprio(1);
+        pv(buf, pb);
+        __builtin_amdgcn_s_setprio(0);
+      }
     }
+    // The odd tiles' state joins the even ones', which hold slot 0: a query's m is finite there. Empty: m = -inf,
+    // l = 0, o = 0, weight 0.
+    float* so = (float*)&Ks[0][0] + qw * (kPfD / 2) * kWave + lane;
+    float* sml = (float*)&Vs[0][0] + qw * 2 * kWave + lane;
+    lds_barrier();
+    if (grp == 1) {
+#pragma unroll
+      for (int dt = 0; dt < kPfD / 32; ++dt)
+#pragma unroll
+        for (int r = 0; r < 16; ++r) so[(dt * 16 + r) * kWave] = o[dt][r];
+      sml[0] = m;
+      sml[kWave] = l;
+    }
+    lds_barrier();
+    if (grp == 1) return;
+    const float m1 = sml[0], c = a.scale * kPfLog2e;
+    const float mm = fmaxf(m, m1);
+    const float w0 = __builtin_amdgcn_exp2f((m - mm) * c), w1 = __builtin_amdgcn_exp2f((m1 - mm) * c);
+    l = l * w0 + sml[kWave] * w1;
+#pragma unroll
+    for (int dt = 0; dt < kPfD / 32; ++dt)
+#pragma unroll
+      for (int r = 0; r < 16; ++r) o[dt][r] = o[dt][r] * w0 + so[(dt * 16 + r) * kWave] * w1;
+  } else {
+    // Wavefronts 4-7 run a phase behind 0-3: in the iteration of tile j they
+    // multiply tile j - 1's p . v first, then tile j's q . k and softmax, so while
+    // the wavefront beside them on their SIMD is in its softmax (VALU) they are in
+    // q . k, and in their softmax it is in p . v (MFMA). V tiles stay for one more
+    // iteration, so V rotates through four LDS buffers and K through three. Every
+    // output accumulator takes the same operations in the same order either way.
+    const bool lag = wave >= kPfWaves / 2;  // wave-uniform
+    u32x4 pprev[4];
+    // Tile j: wait for this wavefront's loads of tile j (tile j + 1's stay in flight), publish them with the
+    // barrier, which also retires every wavefront's reads of K tile j - 1 and V tile j - 2, load tile j + 2 into
+    // those buffers, multiply tile j.
+#pragma unroll 1
+    for (int j = 0; j < nt; ++j) {
+      if (j + 1 < nt)
+        EGPT_WAIT_VMCNT(kTileLoads);
+      else
+        EGPT_WAIT_VMCNT(0);
+      lds_barrier();
+      if (j + 2 < nt) issue(j + 2);
+      const int kbuf = j % 3, vbuf = j % 4;
+      f32x16_pf st[2];
+      // A wavefront raises its issue priority for its MFMA phases, so that where both wavefronts of a SIMD are
+      // ready the one feeding the matrix core goes first and the other's softmax fills in behind it.
+      if (!lag) {
+        u32x4 pb[4];
+        __builtin_amdgcn_s_setprio(1);
+        qk(kbuf, st);
+        __builtin_amdgcn_s_setprio(0);
+        softmax(j, st, pb);
+        __builtin_amdgcn_s_setprio(1);
+        pv(vbuf, pb);
+        __builtin_amdgcn_s_setprio(0);
+      } else {
+        __builtin_amdgcn_s_setprio(1);
+        if (j > 0) pv(vbuf == 0 ? 3 : vbuf - 1, pprev);
+        qk(kbuf, st);
+        __builtin_amdgcn_s_setprio(0);
+        softmax(j, st, pprev);
+      }
+    }
+    if (lag) pv((nt - 1) % 4, pprev);  // tile nt - 1
   }
-  if (lag) pv((nt - 1) % 4, pprev);  // tile nt - 1
 
   // out[tq, hq, 32 dt + 8 (r / 4) + 4 half + r % 4] = o / l, four dims per 8-byte store
   if (tq < a.rows) {
@@ -342,14 +417,21 @@ extern "C" int egpt_prefill_attn(const void* q, int64_t q_ld, const void* k, con
   a.pos0 = pos0;
   // query heads per block: the largest of 4, 2, 1 that divides the group
   a.hb = group % 4 == 0 ? 4 : group % 2 == 0 ? 2 : 1;
-  a.bt = 32 * kPfWaves / a.hb;
-  a.ntiles = (rows + a.bt - 1) / a.bt;
   a.scale = scale;
+  auto blocks = [&](int kvg) {
+    a.bt = 32 * kPfWaves / kvg / a.hb;
+    a.ntiles = (rows + a.bt - 1) / a.bt;
+    return (int64_t)Hkv * (group / a.hb) * a.ntiles;
+  };
+  const int kvg = blocks(1) <= kPfSmallGrid ? 2 : 1;
+  blocks(kvg);
   const dim3 grid((unsigned)(Hkv * (group / a.hb)), (unsigned)a.ntiles);
-  switch (D) {
-    case 32: hipLaunchKernelGGL(prefill_attn_kernel<32>, grid, dim3(kPfThreads), 0, stream, a); break;
-    case 64: hipLaunchKernelGGL(prefill_attn_kernel<64>, grid, dim3(kPfThreads), 0, stream, a); break;
-    default: hipLaunchKernelGGL(prefill_attn_kernel<128>, grid, dim3(kPfThreads), 0, stream, a); break;
-  }
+#define EGPT_PF(DD)                                                                                        \
+  if (kvg == 1) hipLaunchKernelGGL((prefill_attn_kernel<DD, 1>), grid, dim3(kPfThreads), 0, stream, a);    \
+  else hipLaunchKernelGGL((prefill_attn_kernel<DD, 2>), grid, dim3(kPfThreads), 0, stream, a)
+  if (D == 32) { EGPT_PF(32); }
+  else if (D == 64) { EGPT_PF(64); }
+  else { EGPT_PF(128); }
+#undef EGPT_PF
   return EGPT_LAUNCH_STATUS();
 }

@@ -85,6 +85,28 @@ def test_prefill_attention_small_head_dims_long_prompt(d):
     _check(q, k, v, 8, 2, 50)
 
 
+@pytest.mark.parametrize('d', [32, 64, 128])
+@pytest.mark.parametrize('hq,hkv', [(8, 2), (4, 2), (3, 3)])
+@pytest.mark.parametrize('rows,pos0', [(33, 0), (64, 0), (65, 0), (2, 126), (40, 88), (128, 64), (129, 191), (31, 257)])
+def test_prefill_attention_two_tile_groups(d, hq, hkv, rows, pos0):
+    """Small grids, whose wavefronts take the even and the odd tiles: one tile (the second group's state stays empty),
+    odd and even tile counts, a last tile of one slot, first rows that see no odd tile; against the oracle."""
+    q, k, v, _ = _case(rows, hq, hkv, pos0 + rows + 7, pos0, seed=rows + pos0 + d, D=d)
+    _check(q, k, v, hq, hkv, pos0)
+
+
+@pytest.mark.parametrize('d,hq,hkv,rows,pos0', [(32, 8, 2, 4133, 70), (64, 12, 2, 4133, 0), (128, 32, 8, 1100, 33),
+                                                (128, 16, 8, 2100, 0), (128, 8, 8, 4200, 5)])
+def test_prefill_attention_large_and_small_grids_agree(d, hq, hkv, rows, pos0):
+    """A prompt of more than 128 blocks (one group of wavefronts) against the same rows in pieces (two): each is within
+    2^-8 max|v| of the exact value (see above), so they are within 2^-7 of each other."""
+    q, k, v, _ = _case(rows, hq, hkv, pos0 + rows + 9, pos0, seed=rows + d, D=d)
+    whole = _run(q, k, v, hq, hkv, pos0).float()
+    step = 517
+    parts = torch.cat([_run(q[lo:lo + step], k, v, hq, hkv, pos0 + lo) for lo in range(0, rows, step)]).float()
+    assert float((whole - parts).abs().max()) <= 2 ** -7 * float(v.abs().max()) + 2e-4
+
+
 def test_prefill_attention_qwen3_8b_heads_long_prompt():
     # the Qwen3-8B grouping (32 / 8) over a 2048-token prompt: 32 tiles of 64 slots for the last rows
     q, k, v, _ = _case(2048, 32, 8, 2048, 0, seed=11)
