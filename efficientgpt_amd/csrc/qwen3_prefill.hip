@@ -17,6 +17,7 @@ namespace egpt {
 namespace {
 
 constexpr int kThreads = 256;
+typedef uint32_t u32x4_h __attribute__((ext_vector_type(4), aligned(2)));
 
 // Row r of the prompt: x = table[token], h = RMSNorm(x) * w, positions[r] = pos0 + r; block 0 sets *position to the last
 // row's. The sums run in add_rmsnorm_kernel's order (V8: add_rmsnorm_v8_kernel's), so x and h have the bits of
@@ -44,7 +45,7 @@ __global__ __launch_bounds__(kThreads) void prompt_start_kernel(const int64_t* _
   float ss = 0.f;
   if (V8) {
     for (int g = threadIdx.x; g * 8 < n; g += kThreads) {
-      const u32x4 raw = ld16(t + g * 8);
+      const u32x4 raw = *(global_ptr<const u32x4_h>)(t + g * 8);  // the table may start at any element
       *(u32x4*)(xr + g * 8) = raw;
       float v[8];
       Elem<__bf16>::unpack(raw, v);
@@ -188,7 +189,7 @@ extern "C" int egpt_qwen3_prefill(const egpt_qwen3_step* s, const int64_t* token
   const Split sp{ws + l.split, l.split_bytes};
 
   const uint16_t* norm0 = (const uint16_t*)s->layer[0].in_norm;
-  const bool v8 = n % 8 == 0 && ((uintptr_t)s->embed | (uintptr_t)norm0) % 16 == 0;
+  const bool v8 = n % 8 == 0 && (uintptr_t)norm0 % 16 == 0;  // as egpt_rmsnorm chooses over the aligned x and h
   hipLaunchKernelGGL(v8 ? prompt_start_kernel<true> : prompt_start_kernel<false>, dim3(rows), dim3(kThreads),
                      n * sizeof(float), stream, tokens, (const uint16_t*)s->embed, s->vocab, n, norm0, s->eps,
                      (uint16_t*)x, (uint16_t*)h, positions, s->position, (int64_t)pos0);

@@ -167,6 +167,35 @@ def test_prefill_one_call_equals_separate_calls(plen, pos0):
     assert (ta, pa) == (tb, pb) and pa == pos0 + plen
 
 
+@pytest.mark.parametrize('name', ['embed', 'in_w'])
+def test_prefill_one_call_takes_unaligned_weights(name):
+    """An embedding table or first norm that starts off 16-byte alignment (a view into a larger buffer): the first
+    kernel's element order is egpt_rmsnorm's either way, so the bits are those of the separate calls."""
+    from efficientgpt_amd.qwen3 import Qwen3Int8Engine
+    eng, _ = build(SMALL, seed=3, std=0.15, cap=96)
+
+    def shifted(t):
+        flat = torch.empty(t.numel() + 1, dtype=t.dtype, device=t.device)
+        flat[1:] = t.reshape(-1)
+        return flat[1:].view(t.shape)
+
+    packed = {'layers': [dict(L) for L in eng.layers], 'embed': eng.embed, 'norm_w': eng.norm_w, 'head_q': eng.head_q,
+              'head_s': eng.head_s}
+    if name == 'embed':
+        packed['embed'] = shifted(eng.embed)
+    else:
+        packed['layers'][0]['in_w'] = shifted(eng.layers[0]['in_w'])
+    other = Qwen3Int8Engine(eng.cfg, packed, 96, packed=True, inv_freq=eng.inv_freq)
+    assert (other.embed.data_ptr() % 16 != 0) == (name == 'embed')
+    prompt = torch.randint(0, SMALL.vocab, (37,), generator=torch.Generator().manual_seed(1))
+    out = []
+    for fold in (True, False):
+        other.fold_norms = fold
+        other.reset()
+        out.append((other.prefill(prompt).clone(), other.k_cache.clone(), other.v_cache.clone()))
+    assert all(torch.equal(a, b) for a, b in zip(*out))
+
+
 @pytest.mark.parametrize('shape', [SMALL, SMALL8])
 @pytest.mark.parametrize('plen', [40, 128, 4096])
 def test_prefill_folded_norms_equal_separate_calls(shape, plen):
