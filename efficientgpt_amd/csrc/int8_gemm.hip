@@ -651,9 +651,6 @@ int launch_best_tile(const GemmArgs& a, bool swiglu, hipStream_t st) {
 constexpr int kRagBK = 64;
 constexpr int kRagRow = kRagBK + 8;  // bf16 elements per row in LDS
 
-typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
-__device__ __forceinline__ u32x4 ld16_any(const void* p) { return *(global_ptr<const u32x4_b>)p; }
-
 __global__ __launch_bounds__(256) void int8_gemm_ragged_kernel(const GemmArgs a) {
   constexpr int TM = 2, TN = 2, BM = 64, BN = 64;
   __shared__ __align__(16) uint16_t As[2][BM * kRagRow];

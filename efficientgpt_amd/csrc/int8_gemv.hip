@@ -21,6 +21,8 @@
 //   * The row sum is a DPP butterfly over 16 lanes plus four readlanes: a fixed
 //     summation order, so results are bitwise reproducible.
 //   * The scale is applied after the reduction, then one bf16 rounding.
+#include <algorithm>
+
 #include "common.h"
 
 namespace egpt {
@@ -55,34 +57,12 @@ __device__ __forceinline__ void unpack_bf16x16(const u32x4 a, const u32x4 b, flo
   }
 }
 
-// Loads of any alignment, and of the n < 16 (8) elements that a row ends with (zeros after them). An activation of zero
-// cancels its weight's bias, so what a weight's missing bytes hold does not matter.
-typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
-__device__ __forceinline__ u32x4 ld16_any(const void* p) { return *(global_ptr<const u32x4_b>)p; }
-__device__ __forceinline__ u32x4 ld_tail_i8(const int8_t* p, int n) {
-  uint32_t d[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-  for (int e = 0; e < 16; ++e)
-    if (e < n) d[e / 4] |= (uint32_t)(uint8_t)gload(p + e) << (8 * (e % 4));
-  return u32x4{d[0], d[1], d[2], d[3]};
-}
-__device__ __forceinline__ u32x4 ld_tail_bf16(const uint16_t* p, int n) {
-  uint32_t d[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-  for (int e = 0; e < 8; ++e)
-    if (e < n) d[e / 2] |= (uint32_t)gload(p + e) << (16 * (e % 2));
-  return u32x4{d[0], d[1], d[2], d[3]};
-}
-
-// Without RAGGED, preconditions (checked on the host): every K chunk boundary and
+// Fast path. Preconditions (checked on the host): every K chunk boundary and
 // every row start is 16-byte aligned (K % 16 == 0, kchunk % 16 == 0, ldw % 16 == 0,
 // ldx % 8 == 0, aligned base pointers). NCH > 0 means each split covers exactly
 // NCH * kChunk elements, so the chunk loop is fully unrolled with no K masking.
-// RAGGED: any K, strides and base pointers; loads of any alignment, and a row's last
-// partial 16 columns element by element. It replaced a kernel of one element per lane
-// that read every weight row once per activation row (6 x 4001 -> 4096 83 -> 30 us).
 // Rows past N and x rows past m_rows are clamped to valid memory and discarded.
-template <int M, int R, int NCH, int EPI, bool RAGGED = false>
+template <int M, int R, int NCH, int EPI>
 __global__ __launch_bounds__(kGemvThreads) void gemv_i8_rows(
     const uint16_t* __restrict__ x, int64_t ldx, const int8_t* __restrict__ w, int64_t ldw,
     const float* __restrict__ scale, void* __restrict__ out, int64_t ldo, int m_rows, int N, int K,
@@ -115,26 +95,13 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_i8_rows(
   for (int c = 0; c < nch; ++c) {
     const int k = k_begin + c * kChunk + lane * 16;
     if (NCH > 0 || k < k_end) {
-      const bool whole = !RAGGED || k + 16 <= k_end;
       u32x4 wv[R];
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if constexpr (RAGGED)
-          wv[r] = whole ? ld16_any(wrow[r] + k) : ld_tail_i8(wrow[r] + k, k_end - k);
-        else
-          wv[r] = ld16_stream(wrow[r] + k);
-      }
+      for (int r = 0; r < R; ++r) wv[r] = ld16_stream(wrow[r] + k);
 #pragma unroll
       for (int m = 0; m < M; ++m) {
         float xf[16];
-        if constexpr (RAGGED) {
-          if (whole)
-            unpack_bf16x16(ld16_any(xrow[m] + k), ld16_any(xrow[m] + k + 8), xf);
-          else
-            unpack_bf16x16(ld_tail_bf16(xrow[m] + k, k_end - k), ld_tail_bf16(xrow[m] + k + 8, k_end - k - 8), xf);
-        } else {
-          unpack_bf16x16(ld16(xrow[m] + k), ld16(xrow[m] + k + 8), xf);
-        }
+        unpack_bf16x16(ld16(xrow[m] + k), ld16(xrow[m] + k + 8), xf);
         float t = 0.f;
 #pragma unroll
         for (int e = 0; e < 16; ++e) t += xf[e];
@@ -160,6 +127,91 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_i8_rows(
       } else {
         ((float*)out)[((int64_t)blockIdx.y * m_rows + m) * ldo + n] = mine;
       }
+    }
+  }
+}
+
+// Any alignment, strides and K of at least 16 columns per split: one wavefront per output row, 16 columns a lane with
+// loads of any alignment, each weight converted once for up to four activation rows (grid z; 16 rows in one block took
+// 256 registers and left two wavefronts a SIMD: 16 x 520 -> 8192 59 us, in groups of four 21). The codes are converted signed: the
+// biased form above would make x * (w + 128) and 128 * x of an infinite or very large x cancel into NaN, and sums with a
+// mean several times less exact; these kernels keep the plain sum of x * w. The lane that a slice ends in moves its
+// chunk back to end there, with zeros for the activations that the lane before it has.
+template <int M, int EPI>
+__global__ __launch_bounds__(kGemvThreads) void gemv_i8_ragged(
+    const uint16_t* __restrict__ x, int64_t ldx, const int8_t* __restrict__ w, int64_t ldw,
+    const float* __restrict__ scale, void* __restrict__ out, int64_t ldo, int m_rows, int N, int K,
+    int kchunk) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int64_t n = (int64_t)blockIdx.x * kGemvWaves + wave;
+  if (n >= N) return;
+  const uint32_t k_begin = blockIdx.y * (uint32_t)kchunk;
+  const uint32_t k_end = min((uint32_t)K, k_begin + (uint32_t)kchunk);
+  const int m0 = (int)blockIdx.z * M;
+  const int8_t* wr = w + n * ldw;
+  const uint16_t* xr[M];
+  float acc[M];
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    xr[m] = x + (int64_t)min(m0 + m, m_rows - 1) * ldx;
+    acc[m] = 0.f;
+  }
+  for (uint32_t k = k_begin + lane * 16; k < k_end; k += kChunk) {
+    const uint32_t kk = min(k, k_end - 16);
+    const uint32_t skip = k - kk;  // columns of the chunk that the lane before has; 0 but where the slice ends
+    const u32x4 wv = ld16_any(wr + kk);
+    const uint32_t d[4] = {wv.x, wv.y, wv.z, wv.w};
+    float wf[16];
+#pragma unroll
+    for (int e = 0; e < 16; ++e) wf[e] = (float)(int8_t)(d[e / 4] >> (8 * (e % 4)));
+#pragma unroll
+    for (int m = 0; m < M; ++m) {
+      float xf[16];
+      unpack_bf16x16(ld16_any(xr[m] + kk), ld16_any(xr[m] + kk + 8), xf);
+      if (skip) {
+#pragma unroll
+        for (int e = 0; e < 16; ++e) xf[e] = e < (int)skip ? 0.f : xf[e];
+      }
+#pragma unroll
+      for (int e = 0; e < 16; ++e) acc[m] = fmaf(xf[e], wf[e], acc[m]);
+    }
+  }
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+    const float v = wave_sum(acc[m]);
+    if (lane == 0 && m0 + m < m_rows) {
+      if constexpr (EPI == kEpiStore)
+        ((uint16_t*)out)[(int64_t)(m0 + m) * ldo + n] = f32_to_bf16(v * scale[n]);
+      else
+        ((float*)out)[((int64_t)blockIdx.y * m_rows + m0 + m) * ldo + n] = v;
+    }
+  }
+}
+
+// The same for short slices (and K of 0): one element per lane step, every activation row in turn.
+template <int EPI>
+__global__ __launch_bounds__(kGemvThreads) void gemv_i8_short(
+    const uint16_t* __restrict__ x, int64_t ldx, const int8_t* __restrict__ w, int64_t ldw,
+    const float* __restrict__ scale, void* __restrict__ out, int64_t ldo, int m_rows, int N, int K,
+    int kchunk) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int wave = threadIdx.x / kWave;
+  const int64_t n = (int64_t)blockIdx.x * kGemvWaves + wave;
+  if (n >= N) return;
+  const int k_begin = blockIdx.y * kchunk;
+  const int k_end = min(K, k_begin + kchunk);
+  const int8_t* wr = w + n * ldw;
+  for (int m = 0; m < m_rows; ++m) {
+    const uint16_t* xr = x + (int64_t)m * ldx;
+    float a = 0.f;
+    for (int k = k_begin + lane; k < k_end; k += kWave) a = fmaf(bf16_to_f32(xr[k]), (float)wr[k], a);
+    a = wave_sum(a);
+    if (lane == 0) {
+      if constexpr (EPI == kEpiStore)
+        ((uint16_t*)out)[(int64_t)m * ldo + n] = f32_to_bf16(a * scale[n]);
+      else
+        ((float*)out)[((int64_t)blockIdx.y * m_rows + m) * ldo + n] = a;
     }
   }
 }
@@ -605,6 +657,14 @@ __global__ __launch_bounds__(256) void gemv_splitk_reduce(const float* __restric
   y[(int64_t)m * ldy + n] = f32_to_bf16(a * scale[n]);
 }
 
+// Unaligned slices of fewer columns run one element per lane step (gemv_i8_short), whose lanes are then all in use; those
+// of the 16-column form are not, which costs instructions, and these bound calls of more than two rows over enough
+// features for three wavefronts a SIMD. Measured on the MI355X, us, short form / 16-column form: 1 row over 8192 features,
+// K 200 3.65 / 3.69, 257 3.95 / 3.64; 2 rows, 200 4.54 / 4.85, 257 4.97 / 4.87; 5 rows, 257 7.98 / 11.9, 520 11.23 /
+// 11.30; 16 rows, 257 18.3 / 21.5, 520 27.6 / 20.7, 4001 309 / 95; over 2048 features 5 rows, 257 1.21x, 16 rows 1.66x,
+// over 4096 features 5 rows, 257 0.89x, 385 1.04x the short form's speed.
+constexpr int short_k(int rows, int N) { return rows <= 2 || N <= 2048 ? 256 : 512; }
+
 struct GemvArgs {
   const uint16_t* x;
   int64_t ldx;
@@ -616,11 +676,11 @@ struct GemvArgs {
   int m_rows, N, K, kchunk, splits;
 };
 
-template <int M, int R, int NCH, int EPI, bool RAGGED = false>
+template <int M, int R, int NCH, int EPI>
 void launch_rows(const GemvArgs& a, hipStream_t st) {
   const int rows_per_block = kGemvWaves * R;
   dim3 grid((unsigned)((a.N + rows_per_block - 1) / rows_per_block), (unsigned)a.splits);
-  hipLaunchKernelGGL((gemv_i8_rows<M, R, NCH, EPI, RAGGED>), grid, dim3(kGemvThreads), 0, st, a.x, a.ldx, a.w, a.ldw,
+  hipLaunchKernelGGL((gemv_i8_rows<M, R, NCH, EPI>), grid, dim3(kGemvThreads), 0, st, a.x, a.ldx, a.w, a.ldw,
                      a.scale, a.out, a.ldo, a.m_rows, a.N, a.K, a.kchunk);
 }
 
@@ -665,12 +725,15 @@ int launch_gemv(const GemvArgs& a, hipStream_t st) {
                        ((uintptr_t)a.w % 16 == 0) && ((uintptr_t)a.x % 16 == 0) &&
                        (a.m_rows == 1 || a.ldx % 8 == 0);
   if (!aligned || a.K == 0) {
-    // one row per wavefront: the conversions of a weight feed up to 16 rows, and these calls are small
-    if (a.m_rows == 1) launch_rows<1, 1, 0, EPI, true>(a, st);
-    else if (a.m_rows <= 2) launch_rows<2, 1, 0, EPI, true>(a, st);
-    else if (a.m_rows <= 4) launch_rows<4, 1, 0, EPI, true>(a, st);
-    else if (a.m_rows <= 8) launch_rows<8, 1, 0, EPI, true>(a, st);
-    else launch_rows<16, 1, 0, EPI, true>(a, st);
+    const unsigned bx = (unsigned)(((int64_t)a.N + kGemvWaves - 1) / kGemvWaves), by = (unsigned)a.splits;
+#define EGPT_UNALIGNED(GROUPS, ...)                                                                             \
+  hipLaunchKernelGGL((__VA_ARGS__), dim3(bx, by, (unsigned)(GROUPS)), dim3(kGemvThreads), 0, st, a.x, a.ldx, a.w, \
+                     a.ldw, a.scale, a.out, a.ldo, a.m_rows, a.N, a.K, a.kchunk)
+    if (std::min(a.K, a.kchunk) < short_k(a.m_rows, a.N)) { EGPT_UNALIGNED(1, gemv_i8_short<EPI>); }
+    else if (a.m_rows == 1) { EGPT_UNALIGNED(1, gemv_i8_ragged<1, EPI>); }
+    else if (a.m_rows <= 2) { EGPT_UNALIGNED(1, gemv_i8_ragged<2, EPI>); }
+    else { EGPT_UNALIGNED((a.m_rows + 3) / 4, gemv_i8_ragged<4, EPI>); }
+#undef EGPT_UNALIGNED
     return EGPT_LAUNCH_STATUS();
   }
   // Exact chunk count per split when every split has the same length.

@@ -446,6 +446,81 @@ def test_shapes_and_alignments_of_no_kind(m, k, n):
     assert bool((y[:, n:] == -7).all())
 
 
+def _unaligned(x, q, s):
+    """Device copies of x [m, k] and q [n, k] whose rows lie off every 16-byte boundary, between values that would show."""
+    xb = torch.full((x.shape[0], x.shape[1] + 3), float('nan'), dtype=torch.bfloat16)
+    xb[:, 1:x.shape[1] + 1] = x
+    qb = torch.full((q.shape[0], q.shape[1] + 5), 119, dtype=torch.int8)
+    qb[:, 3:q.shape[1] + 3] = q
+    return xb.cuda()[:, 1:x.shape[1] + 1], qb.cuda()[:, 3:q.shape[1] + 3], s.cuda()
+
+
+def _unaligned_gemv(x, q, s, splits):
+    """The decode GEMV of unaligned rows (splits 0), or its split form: (output, fp32 partial sums [splits, m, n])."""
+    from efficientgpt_amd import _lib
+    lib = _lib.lib()
+    (m, k), n = x.shape, q.shape[0]
+    xd, qd, sd = _unaligned(x, q, s)
+    y = torch.full((m, n), -7.0, device='cuda', dtype=torch.bfloat16)
+    part = torch.zeros(max(splits, 1), m, n, device='cuda')
+    args = (xd.data_ptr(), xd.stride(0), qd.data_ptr(), qd.stride(0), sd.data_ptr(), y.data_ptr(), n, m, n, k)
+    if splits:
+        st = lib.egpt_int8_gemv_splitk(*args, splits, part.data_ptr(), part.numel() * 4, _lib.stream_ptr())
+    else:
+        st = lib.egpt_int8_gemv(*args, _lib.stream_ptr())
+    assert st == 0
+    return y, part
+
+
+@pytest.mark.parametrize('splits', [0, 3])
+@pytest.mark.parametrize('m', [1, 2, 5, 16])
+@pytest.mark.parametrize('k', [40, 1040, 4001])
+def test_unaligned_rows_with_infinite_nan_and_large_activations(m, k, splits):
+    """An infinity, a NaN or a finite value near the top of the range in the last activation row: its outputs are the
+    formula's (inf * 0 is NaN, inf * w is inf with w's sign, 3e36 * w stays finite), the other rows' those of finite
+    rows, and a weight row of zeros gives exactly zero under activations with a mean."""
+    n = 24
+    x, q, s = make_case(m, k, n, seed=m + k)
+    x = (x.float() + 3).to(torch.bfloat16)
+    q.clamp_(-100, 100)
+    q[7] = 0
+    base, _ = _unaligned_gemv(x, q, s, splits)
+    assert bool((base[:, 7] == 0).all())
+    for j in (0, k // 2, k - 1):
+        q[:, j] = torch.tensor([5, -5, 0, 1, -1, 100, -100, 0] * 3, dtype=torch.int8)
+        finite, _ = _unaligned_gemv(x, q, s, splits)
+        for value in (float('inf'), float('-inf'), float('nan'), 3e36):
+            xs = x.clone()
+            xs[m - 1, j] = value
+            y, _ = _unaligned_gemv(xs, q, s, splits)
+            assert torch.equal(y[:m - 1], finite[:m - 1])
+            # infinities of both signs never meet in a row, so the exact value is that of any order
+            want = (xs[m - 1].double()[None] * q.double()).sum(1) * s.double()
+            got = y[m - 1].cpu().double()
+            assert torch.equal(torch.isnan(got), torch.isnan(want)), (value, j)
+            ok = ~torch.isnan(want)
+            inf = ok & torch.isinf(want)
+            assert torch.equal(got[inf], want[inf])
+            big = ok & ~torch.isinf(want) & (want.abs() > 1e20)
+            # one rounding to bf16 of an fp32 value
+            assert bool(((got - want).abs()[big] <= 2.0 ** -8 * (1 + 2.0 ** -10) * want.abs()[big]).all()), (value, j)
+
+
+@pytest.mark.parametrize('m,k,n', [(m, k, 200) for m in (1, 2, 5, 16) for k in (255, 257, 300, 4001, 9001)] +
+                         [(2, 513, 2100), (3, 511, 2100), (3, 513, 2100), (16, 511, 2100), (16, 527, 2100)])
+def test_unaligned_rows_fp32_sums_are_as_exact_as_a_plain_sum(m, k, n):
+    """The fp32 sums behind the rounding to bf16 (the partials of one split) against 64 bits, activations with a mean of
+    3. A lane adds about k / 64 products one after the other and six additions join the lanes; each step rounds a partial
+    sum, which grows like a random walk, by at most 2^-24, so the error's 2-norm is below 2^-24 sqrt(k / 128 + 6) of the
+    result's. A form that adds and then removes 128 * sum(x) rounds sums many times larger."""
+    x, q, s = make_case(m, k, n, seed=m + k)
+    x = (x.float() + 3).to(torch.bfloat16)
+    _, part = _unaligned_gemv(x, q, s, 1)
+    want = x.double() @ q.double().t()
+    err = float((part[0].cpu().double() - want).norm() / want.norm())
+    assert err <= 2.0 ** -24 * (k / 128 + 6) ** 0.5, err
+
+
 def test_prefill_op_keeps_leading_dims():
     from efficientgpt_amd.int8_linear import int8_linear
     x, q, s = make_case(48, 2048, 512, seed=11)
