@@ -650,6 +650,10 @@ int launch_best_tile(const GemmArgs& a, bool swiglu, hipStream_t st) {
 // 54 now; 500 x 7001 -> 8000 19055 -> 159, 40 x 7001 -> 8000 955 -> 81.
 constexpr int kRagBK = 64;
 constexpr int kRagRow = kRagBK + 8;  // bf16 elements per row in LDS
+// Steps of a row and a step's first column, for any int K (two steps past the last are asked for).
+constexpr int rag_steps(int K) { return (int)(((int64_t)K + kRagBK - 1) / kRagBK); }
+constexpr int64_t rag_column(int kt) { return (int64_t)kt * kRagBK; }
+static_assert(rag_steps(INT32_MAX) == 1 << 25 && rag_column(rag_steps(INT32_MAX) + 1) > INT32_MAX, "");
 
 __global__ __launch_bounds__(256) void int8_gemm_ragged_kernel(const GemmArgs a) {
   constexpr int TM = 2, TN = 2, BM = 64, BN = 64;
@@ -670,10 +674,10 @@ __global__ __launch_bounds__(256) void int8_gemm_ragged_kernel(const GemmArgs a)
 #pragma unroll
   for (int j = 0; j < 2; ++j) xp[j] = a.x + min(m0 + 32 * j + tid / 8, (int64_t)a.M - 1) * a.ldx + xc;
   const int8_t* wp = a.w + min(n0 + tid / 4, (int64_t)a.N - 1) * a.ldw + wc;
-  const int nk = (a.K + kRagBK - 1) / kRagBK;
+  const int nk = rag_steps(a.K);
   u32x4 xr[2][2], wr[2];
   auto load_step = [&](int kt, int set) {
-    const int k0 = kt * kRagBK;
+    const int64_t k0 = rag_column(kt);
     if (k0 + kRagBK <= a.K) {
 #pragma unroll
       for (int j = 0; j < 2; ++j) xr[set][j] = ld16_any(xp[j] + k0);
