@@ -644,21 +644,20 @@ int launch_best_tile(const GemmArgs& a, bool swiglu, hipStream_t st) {
 
 // Any K, alignment and size: 64 x 64 of y per block, four wavefronts as 2 x 2. The tiles above need 16-byte aligned rows
 // for their loads into LDS and K in whole steps; here both operands go through registers with loads of any alignment,
-// 64 K columns a step and two steps ahead, and into LDS as bf16 (rows padded by 16 bytes against bank conflicts). The
-// columns past K of a last step are loaded element by element as zeros. Rows past M or N read the last one.
-// It replaced a vector kernel (one wavefront per feature and 4 rows, 2-byte loads): 300 x 4001 -> 4096 1749 us before,
-// 54 now; 500 x 7001 -> 8000 19055 -> 159, 40 x 7001 -> 8000 955 -> 81.
-constexpr int kRagBK = 64;
-constexpr int kRagRow = kRagBK + 8;  // bf16 elements per row in LDS
-// Steps of a row and a step's first column, for any int K (two steps past the last are asked for).
-constexpr int rag_steps(int K) { return (int)(((int64_t)K + kRagBK - 1) / kRagBK); }
-constexpr int64_t rag_column(int kt) { return (int64_t)kt * kRagBK; }
-static_assert(rag_steps(INT32_MAX) == 1 << 25 && rag_column(rag_steps(INT32_MAX) + 1) > INT32_MAX, "");
+// BK (64 or 128) K columns a step and two steps ahead, and into LDS as bf16 (rows padded by 16 bytes against bank
+// conflicts). Rows past M or N read the last one. Against the vector kernel below, us: 300 x 4001 -> 4096 1749 -> 47, 500 x
+// 7001 -> 8000 19055 -> 146, 40 x 7001 -> 8000 955 -> 64.
+constexpr int64_t rag_column(int kt, int BK) { return (int64_t)kt * BK; }  // a step's first, for any int K
+static_assert(rag_column(INT32_MAX / 64 + 2, 64) > INT32_MAX, "");
 
+template <int BK>
 __global__ __launch_bounds__(256) void int8_gemm_ragged_kernel(const GemmArgs a) {
   constexpr int TM = 2, TN = 2, BM = 64, BN = 64;
-  __shared__ __align__(16) uint16_t As[2][BM * kRagRow];
-  __shared__ __align__(16) uint16_t Bs[2][BN * kRagRow];
+  constexpr int kRow = BK + 8;                            // bf16 elements per row in LDS
+  constexpr int kXT = BK / 8, kWT = BK / 16;              // threads per x row, per weight row
+  constexpr int kXL = BM * kXT / 256, kWL = BN * kWT / 256;  // 16-byte loads per thread and step
+  __shared__ __align__(16) uint16_t As[2][BM * kRow];
+  __shared__ __align__(16) uint16_t Bs[2][BN * kRow];
   const int tid = threadIdx.x;
   const int lane = tid & (kWave - 1);
   const int wave = tid / kWave;
@@ -667,94 +666,178 @@ __global__ __launch_bounds__(256) void int8_gemm_ragged_kernel(const GemmArgs a)
   gemm_tile((int)blockIdx.x, a.tiles_m, a.tiles_n, pid_m, pid_n);
   const int64_t m0 = (int64_t)pid_m * BM, n0 = (int64_t)pid_n * BN;
 
-  // this thread's chunks of a step: x rows tid / 8 and 32 + tid / 8, 8 columns from 8 (tid % 8); weight row tid / 4, 16
-  // columns from 16 (tid % 4)
-  const int xc = 8 * (tid % 8), wc = 16 * (tid % 4);
-  const uint16_t* xp[2];
+  // this thread's chunks of a step: 8 columns of x rows tid / kXT + j 256 / kXT, 16 columns of weight rows likewise
+  const int xc = 8 * (tid % kXT), wc = 16 * (tid % kWT);
+  const uint16_t* xp[kXL];
+  const int8_t* wp[kWL];
 #pragma unroll
-  for (int j = 0; j < 2; ++j) xp[j] = a.x + min(m0 + 32 * j + tid / 8, (int64_t)a.M - 1) * a.ldx + xc;
-  const int8_t* wp = a.w + min(n0 + tid / 4, (int64_t)a.N - 1) * a.ldw + wc;
-  const int nk = rag_steps(a.K);
-  u32x4 xr[2][2], wr[2];
-  auto load_step = [&](int kt, int set) {
-    const int64_t k0 = rag_column(kt);
-    if (k0 + kRagBK <= a.K) {
+  for (int j = 0; j < kXL; ++j)
+    xp[j] = a.x + min(m0 + 256 / kXT * j + tid / kXT, (int64_t)a.M - 1) * a.ldx + xc;
 #pragma unroll
-      for (int j = 0; j < 2; ++j) xr[set][j] = ld16_any(xp[j] + k0);
-      wr[set] = ld16_any(wp + k0);
-    } else if (k0 < a.K) {
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        uint32_t d[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          if (k0 + xc + e < a.K) d[e / 2] |= (uint32_t)gload(xp[j] + k0 + e) << (16 * (e % 2));
-        xr[set][j] = u32x4{d[0], d[1], d[2], d[3]};
-      }
-      uint32_t d[4] = {0u, 0u, 0u, 0u};
-#pragma unroll
-      for (int e = 0; e < 16; ++e)
-        if (k0 + wc + e < a.K) d[e / 4] |= (uint32_t)(uint8_t)gload(wp + k0 + e) << (8 * (e % 4));
-      wr[set] = u32x4{d[0], d[1], d[2], d[3]};
-    }
+  for (int j = 0; j < kWL; ++j) wp[j] = a.w + min(n0 + 256 / kWT * j + tid / kWT, (int64_t)a.N - 1) * a.ldw + wc;
+  const int nk = a.K / BK;  // whole steps
+  struct Regs {
+    u32x4 x[kXL], w[kWL];
   };
-  auto store_step = [&](int buf, int set) {
+  auto load = [&](Regs& r, int64_t k0) {
 #pragma unroll
-    for (int j = 0; j < 2; ++j) *(u32x4*)&As[buf][(32 * j + tid / 8) * kRagRow + xc] = xr[set][j];
-    bf16x8* b = (bf16x8*)&Bs[buf][(tid / 4) * kRagRow + wc];
-    b[0] = int8x8_to_bf16(wr[set].x, wr[set].y);
-    b[1] = int8x8_to_bf16(wr[set].z, wr[set].w);
+    for (int j = 0; j < kXL; ++j) r.x[j] = ld16_any(xp[j] + k0);
+#pragma unroll
+    for (int j = 0; j < kWL; ++j) r.w[j] = ld16_any(wp[j] + k0);
+  };
+  auto store = [&](const Regs& r, int buf) {
+#pragma unroll
+    for (int j = 0; j < kXL; ++j) *(u32x4*)&As[buf][(256 / kXT * j + tid / kXT) * kRow + xc] = r.x[j];
+#pragma unroll
+    for (int j = 0; j < kWL; ++j) {
+      bf16x8* b = (bf16x8*)&Bs[buf][(256 / kWT * j + tid / kWT) * kRow + wc];
+      b[0] = int8x8_to_bf16(r.w[j].x, r.w[j].y);
+      b[1] = int8x8_to_bf16(r.w[j].z, r.w[j].w);
+    }
   };
 
   const int r16 = lane % 16, h = lane / 16;
-  const int arow = (wm0 + r16) * kRagRow + 8 * h;
-  const int brow = (wn0 + 4 * TN * (r16 / 4) + r16 % 4) * kRagRow + 8 * h;
+  const int arow = (wm0 + r16) * kRow + 8 * h;
+  const int brow = (wn0 + 4 * TN * (r16 / 4) + r16 % 4) * kRow + 8 * h;
   f32x4 acc[TM][TN];
 #pragma unroll
   for (int tm = 0; tm < TM; ++tm)
 #pragma unroll
     for (int tn = 0; tn < TN; ++tn) acc[tm][tn] = f32x4{};
-  // Step kt from LDS buffer and register set kt % 2: its loads' successors go out first, then its MFMAs, then the next
-  // step's data into the other buffer.
-  auto step = [&](int kt, int cur) {
-    load_step(kt + 2, cur);
-    __builtin_amdgcn_sched_barrier(0);
-    bf16x8 xf[2][TM], wf[2][TN];
+  auto mma = [&](int buf) {
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks) {
+    for (int k2 = 0; k2 < BK / 64; ++k2) {
+      bf16x8 xf[2][TM], wf[2][TN];
 #pragma unroll
-      for (int tm = 0; tm < TM; ++tm) xf[ks][tm] = *(const bf16x8*)&As[cur][arow + tm * 16 * kRagRow + 32 * ks];
+      for (int ks = 0; ks < 2; ++ks) {
 #pragma unroll
-      for (int tn = 0; tn < TN; ++tn) wf[ks][tn] = *(const bf16x8*)&Bs[cur][brow + tn * 4 * kRagRow + 32 * ks];
-    }
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-#pragma unroll
-      for (int tm = 0; tm < TM; ++tm)
+        for (int tm = 0; tm < TM; ++tm)
+          xf[ks][tm] = *(const bf16x8*)&As[buf][arow + tm * 16 * kRow + 64 * k2 + 32 * ks];
 #pragma unroll
         for (int tn = 0; tn < TN; ++tn)
-          acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][tn], xf[ks][tm], acc[tm][tn], 0, 0, 0);
-    if (kt + 1 < nk) store_step(1 - cur, 1 - cur);
+          wf[ks][tn] = *(const bf16x8*)&Bs[buf][brow + tn * 4 * kRow + 64 * k2 + 32 * ks];
+      }
+#pragma unroll
+      for (int ks = 0; ks < 2; ++ks)
+#pragma unroll
+        for (int tm = 0; tm < TM; ++tm)
+#pragma unroll
+          for (int tn = 0; tn < TN; ++tn)
+            acc[tm][tn] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(wf[ks][tn], xf[ks][tm], acc[tm][tn], 0, 0, 0);
+    }
+  };
+  // Step kt from LDS buffer and register set kt % 2: its loads' successors go out first, then its MFMAs, then the next
+  // step's data into the other buffer.
+  Regs r0, r1;
+  auto step = [&](int kt, int cur, Regs& mine, const Regs& next) {
+    if (kt + 2 < nk) load(mine, rag_column(kt + 2, BK));
+    __builtin_amdgcn_sched_barrier(0);
+    mma(cur);
+    if (kt + 1 < nk) store(next, 1 - cur);
     __builtin_amdgcn_sched_barrier(0);
     lds_barrier();
   };
-  load_step(0, 0);
-  load_step(1, 1);
-  if (nk > 0) store_step(0, 0);
-  lds_barrier();
-  for (int kt = 0; kt < nk; kt += 2) {
-    step(kt, 0);
-    if (kt + 1 < nk) step(kt + 1, 1);
+  if (nk > 0) {
+    load(r0, 0);
+    if (nk > 1) load(r1, BK);
+    store(r0, 0);
+    lds_barrier();
+    for (int kt = 0; kt < nk; kt += 2) {
+      step(kt, 0, r0, r1);
+      if (kt + 1 < nk) step(kt + 1, 1, r1, r0);
+    }
+  }
+  const int left = a.K % BK;
+  if (left) {  // the columns past the last whole step
+    Regs r;
+    if (nk > 0) {
+      // the BK columns before K, with zeros for the activations already added
+      load(r, (int64_t)a.K - BK);
+      u32x4 mask;
+#pragma unroll
+      for (int i = 0; i < 4; ++i)
+        mask[i] = (xc + 2 * i >= BK - left ? 0xffffu : 0u) | (xc + 2 * i + 1 >= BK - left ? 0xffff0000u : 0u);
+#pragma unroll
+      for (int j = 0; j < kXL; ++j) r.x[j] &= mask;
+    } else {  // a row shorter than a step: element by element, zeros after it
+#pragma unroll
+      for (int j = 0; j < kXL; ++j) {
+        uint32_t d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          if (xc + e < left) d[e / 2] |= (uint32_t)gload(xp[j] + e) << (16 * (e % 2));
+        r.x[j] = u32x4{d[0], d[1], d[2], d[3]};
+      }
+#pragma unroll
+      for (int j = 0; j < kWL; ++j) {
+        uint32_t d[4] = {0u, 0u, 0u, 0u};
+#pragma unroll
+        for (int e = 0; e < 16; ++e)
+          if (wc + e < left) d[e / 4] |= (uint32_t)(uint8_t)gload(wp[j] + e) << (8 * (e % 4));
+        r.w[j] = u32x4{d[0], d[1], d[2], d[3]};
+      }
+    }
+    store(r, 0);
+    lds_barrier();
+    mma(0);
   }
   gemm_store_rows<TM, TN, false>(a, acc, m0 + wm0 + r16, n0 + wn0 + 4 * TN * h);
 }
 
+// The same for short rows and small outputs: one wavefront per feature n and group of kVectorRows rows, lanes striding K
+// one element at a time, fp32 sums reduced across the wavefront in a fixed order.
+constexpr int kVectorRows = 4;
+constexpr int kVectorWaves = 4;
+
+__global__ __launch_bounds__(kVectorWaves * kWave) void int8_gemm_vector_kernel(
+    const uint16_t* __restrict__ x, int64_t ldx, const int8_t* __restrict__ w, int64_t ldw,
+    const float* __restrict__ scale, uint16_t* __restrict__ y, int64_t ldy, int M, int N, int K) {
+  const int lane = threadIdx.x & (kWave - 1);
+  const int64_t mgroups = ((int64_t)M + kVectorRows - 1) / kVectorRows;
+  const int64_t wv = (int64_t)blockIdx.x * kVectorWaves + threadIdx.x / kWave;
+  if (wv >= mgroups * N) return;   // wave-uniform
+  const int64_t n = wv / mgroups;  // neighbouring wavefronts share a weight row
+  const int64_t m0 = (wv - n * mgroups) * kVectorRows;
+  const int8_t* wr = w + n * ldw;
+  float acc[kVectorRows] = {};
+  for (int64_t k = lane; k < K; k += kWave) {
+    const float wk = (float)gload(wr + k);
+#pragma unroll
+    for (int r = 0; r < kVectorRows; ++r)
+      if (m0 + r < M) acc[r] = fmaf(bf16_to_f32(gload(x + (m0 + r) * ldx + k)), wk, acc[r]);
+  }
+#pragma unroll
+  for (int r = 0; r < kVectorRows; ++r) {
+    const float sum = wave_sum(acc[r]);
+    if (lane == r && m0 + r < M) gstore(y + (m0 + r) * ldy + n, f32_to_bf16(bf16_to_f32(f32_to_bf16(sum)) * scale[n]));
+  }
+}
+
+// Outputs up to which the vector kernel is the faster one. Measured on the MI355X, us, vector / tiles: K below one step,
+// which the tiles load element by element, 64 x 20 -> 300 4.5 / 5.6, 128 x 20 -> 300 5.8 / 5.7; short rows, 32 x 257 -> 64
+// 5.2 / 5.7, 128 x 257 -> 128 5.9 / 5.8; 64 x 520 -> 64 7.2 / 6.4.
+constexpr int64_t vector_outputs(int K) { return K < 64 ? 32768 : K < 512 ? 10240 : 0; }
+
+// Steps of 128 columns where the tiles are at most two a CU (70 KiB of LDS each) and a row is several steps long: 17 x
+// 8191 -> 1000 70 -> 57 us, 200 x 8191 -> 8192 96 -> 91; 17 x 520 -> 300 6.5 -> 6.8; 1024 tiles, 512 x 8191 -> 8192, 5% slower.
+constexpr int64_t kRagWideTiles = 512;
+constexpr int kRagWideK = 768;
+
 int launch_ragged(GemmArgs a, hipStream_t st) {
+  if ((int64_t)a.M * a.N <= vector_outputs(a.K)) {
+    const int64_t waves = ((int64_t)a.M + kVectorRows - 1) / kVectorRows * a.N;
+    hipLaunchKernelGGL(int8_gemm_vector_kernel, dim3((unsigned)((waves + kVectorWaves - 1) / kVectorWaves)),
+                       dim3(kVectorWaves * kWave), 0, st, a.x, a.ldx, a.w, a.ldw, a.scale, a.y, a.ldy, a.M, a.N, a.K);
+    return EGPT_LAUNCH_STATUS();
+  }
   const int64_t tm = ((int64_t)a.M + 63) / 64, tn = ((int64_t)a.N + 63) / 64;
   if (tm * tn > (int64_t)INT32_MAX) return EGPT_ERR_UNSUPPORTED;
   a.tiles_m = (int)tm;
   a.tiles_n = (int)tn;
-  hipLaunchKernelGGL(int8_gemm_ragged_kernel, dim3((unsigned)(tm * tn)), dim3(256), 0, st, a);
+  if (tm * tn <= kRagWideTiles && a.K >= kRagWideK)
+    hipLaunchKernelGGL(int8_gemm_ragged_kernel<128>, dim3((unsigned)(tm * tn)), dim3(256), 0, st, a);
+  else
+    hipLaunchKernelGGL(int8_gemm_ragged_kernel<64>, dim3((unsigned)(tm * tn)), dim3(256), 0, st, a);
   return EGPT_LAUNCH_STATUS();
 }
 

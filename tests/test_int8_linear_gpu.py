@@ -521,6 +521,36 @@ def test_unaligned_rows_fp32_sums_are_as_exact_as_a_plain_sum(m, k, n):
     assert err <= 2.0 ** -24 * (k / 128 + 6) ** 0.5, err
 
 
+@pytest.mark.parametrize('m,k,n', [(17, 20, 1927), (17, 20, 1928), (17, 63, 1928), (100, 64, 102), (100, 64, 103),
+                                   (100, 65, 103), (100, 127, 103), (20, 511, 512), (20, 511, 513), (20, 512, 10),
+                                   (65, 767, 300), (65, 768, 300), (65, 769, 300), (65, 896, 300), (130, 1000, 200),
+                                   (70, 1151, 170), (40, 777, 32769)])
+def test_unaligned_prompt_rows_at_the_edges_of_each_form(m, k, n):
+    """The prefill GEMM of unaligned rows on each side of its rules (outputs of the vector form, steps of 64 and 128
+    columns, last steps of every kind), with an infinity and a NaN just outside each row: the oracle's formula; an infinity
+    inside a row reaches exactly that row's outputs, with its weights' signs."""
+    from efficientgpt_amd import _lib
+    lib = _lib.lib()
+    x, q, s = make_case(m, k, n, seed=m + k + n)
+    xd, qd, sd = _unaligned(x, q, s)
+    y = torch.full((m, n), -7.0, device='cuda', dtype=torch.bfloat16)
+
+    def run():
+        assert lib.egpt_int8_gemm(xd.data_ptr(), k + 3, qd.data_ptr(), k + 5, sd.data_ptr(), y.data_ptr(), n, m, n, k,
+                                  _lib.stream_ptr()) == 0
+        return y.clone()
+
+    first = run()
+    check_against_oracle(first.cpu(), x, q, s)
+    for j in (0, k // 64 * 64 - 1, k - 1):
+        xd[m - 1, j] = float('inf')
+        got = run()
+        xd[m - 1, j] = x[m - 1, j].item()
+        assert torch.equal(got[:m - 1], first[:m - 1])
+        want = torch.where(qd[:, j] == 0, float('nan'), qd[:, j].sign() * float('inf'))
+        assert torch.equal(torch.nan_to_num(got[m - 1].float(), 7.0), torch.nan_to_num(want, 7.0))
+
+
 def test_prefill_op_keeps_leading_dims():
     from efficientgpt_amd.int8_linear import int8_linear
     x, q, s = make_case(48, 2048, 512, seed=11)
