@@ -211,8 +211,8 @@ class Qwen3Int8Engine:
 
         # Prompt passes run from one call (egpt_qwen3_prefill), which folds the residual add + RMSNorm after o_proj and
         # down_proj into the split-K GEMM's reduce, q/k norm + RoPE into the split-K QKV reduce and SwiGLU into the
-        # gate/up GEMM; False runs a call per op instead: egpt_embed, the norms, the linears, egpt_qk_norm_rope,
-        # egpt_silu_mul (the same bits).
+        # gate/up GEMM; False (and a pass over replaced tensors) runs a call per op instead: egpt_embed, the norms, the
+        # linears, egpt_qk_norm_rope, egpt_silu_mul (the same bits).
         self.fold_norms = True
         pk = weights if packed else pack_qwen3(c, weights)
         check_packed(c, pk)
@@ -309,6 +309,13 @@ class Qwen3Int8Engine:
         if self._ring_dev:
             d.token_ring, d.token_ring_slots = self._ring_dev, self.cap
         self._step_c = d
+        self._step_tensors = self._tensor_addresses()
+
+    def _tensor_addresses(self):
+        """The addresses of the tensors a prompt pass reads and writes, as the engine holds them now."""
+        held = (self.embed, self.norm_w, self.head_q, self.head_s, self.cos, self.sin, self.k_cache, self.v_cache,
+                self.token, self.position, self.logits)
+        return [t.data_ptr() for t in held] + [t.data_ptr() for L in self.layers for t in L.values()]
 
     # ------------------------------------------------------------------ construction helpers
 
@@ -519,7 +526,9 @@ class Qwen3Int8Engine:
         if pos0 + t > self.cap:
             raise ValueError('prompt exceeds the cache capacity')
         lib = _lib.lib()
-        if self.fold_norms:
+        # The descriptor holds the addresses the engine was built with. Where a tensor has been replaced since (a layer's
+        # weight, the cache), the calls below take the tensors themselves, with the strides they have.
+        if self.fold_norms and self._tensor_addresses() == self._step_tensors:
             need = ctypes.c_size_t()
             _lib.check('egpt_qwen3_prefill_workspace', lib.egpt_qwen3_prefill_workspace(ctypes.byref(self._step_c), t,
                                                                                         ctypes.byref(need)))

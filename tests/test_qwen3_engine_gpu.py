@@ -196,6 +196,32 @@ def test_prefill_one_call_takes_unaligned_weights(name):
     assert all(torch.equal(a, b) for a, b in zip(*out))
 
 
+@pytest.mark.parametrize('plen', [1, 20, 100])
+def test_prefill_reads_the_tensors_the_engine_holds(plen):
+    """Weights, norms, embedding, head and caches replaced on a built engine (the former ones stay alive) take effect in
+    the next prompt pass: the logits and caches of an engine built with them, bit for bit."""
+    eng, _ = build(SMALL, seed=3, std=0.15, cap=256)
+    other, _ = build(SMALL, seed=4, std=0.15, cap=256)
+    prompt = torch.randint(0, SMALL.vocab, (plen,), generator=torch.Generator().manual_seed(plen))
+    want = other.prefill(prompt).clone()
+    assert not torch.equal(eng.prefill(prompt), want)
+    former = [eng.embed, eng.norm_w, eng.head_q, eng.head_s, eng.k_cache, eng.v_cache, eng.layers]
+    eng.layers = [{k: v.clone() for k, v in L.items()} for L in other.layers]
+    eng.embed, eng.norm_w = other.embed.clone(), other.norm_w.clone()
+    eng.head_q, eng.head_s = other.head_q.clone(), other.head_s.clone()
+    eng.k_cache, eng.v_cache = torch.zeros_like(eng.k_cache), torch.zeros_like(eng.v_cache)
+    assert torch.equal(eng.prefill(prompt), want)
+    assert torch.equal(eng.k_cache, other.k_cache) and torch.equal(eng.v_cache, other.v_cache)
+    # one weight of one layer
+    L = eng.layers[-1]
+    former.append(L['down_s'])
+    L['down_s'] = L['down_s'] * 2
+    changed = eng.prefill(prompt).clone()
+    assert not torch.equal(changed, want)
+    eng.fold_norms = False
+    assert torch.equal(eng.prefill(prompt), changed)
+
+
 @pytest.mark.parametrize('shape', [SMALL, SMALL8])
 @pytest.mark.parametrize('plen', [40, 128, 4096])
 def test_prefill_folded_norms_equal_separate_calls(shape, plen):
