@@ -892,33 +892,27 @@ int launch_r(const FusedGemv& a, int nch, unsigned blocks, hipStream_t st) {
 }
 
 // Blocks of a fused GEMV launch: one tile per wavefront, except the lm_head,
-// whose grid is capped at two to four 8-wave blocks per CU, so each block stages
-// and normalises the activation once and reduces its argmax once over many tiles:
-// two where the rows are long (the prologue grows with them), four where not.
-// Measured on the MI355X (us, a decode step of four Qwen3-1.7B layers, K 2048 / of
-// two Qwen3-8B layers, K 4096, the head 311 / 622 MB of it): 256 blocks 153.6 /
-// 218.6, 384 152.5 / 237, 512 150.8 / 219.5, 640 157.8 / 231.4, 768 154.6 / 222.4,
-// 1024 150.8 / 224.5, 1280 152.0 / 226.5, uncapped 187 / 300; in another setting
-// 512 and 1024 gave 153.1 and 152.0 / 213.7 and 217.4. Grids that give every
-// wavefront the same number of tiles were no better (512: 150.3 / 220.9).
-constexpr unsigned head_max_blocks(int K) { return K > 2048 ? 512 : 1024; }
+// whose grid is capped (about four 8-wave blocks per CU) so each block stages
+// the activation once and reduces its argmax once over many tiles. The cap does
+// not depend on K: egpt_int8_gemv_fused_parts takes a description with K unset.
+// Measured on the MI355X, the head alone at 151936 features, us, 1024 blocks / 512:
+// K 2560 63.0 / 63.0, 3072 71.1 / 73.5, 4096 100.2 / 97.1, 5120 121.1 / 125.2; at
+// 128256, 8192 158.8 / 162.8; uncapped, a step of two Qwen3-8B layers took 300
+// against 224.
+constexpr unsigned kHeadMaxBlocks = 1024;
 
-unsigned gemv_blocks(int64_t n, bool pairs) {
+unsigned gemv_blocks(int64_t n, bool pairs, bool capped) {
   const int rh = features_per_wave(n, pairs);
   const int64_t tiles = (n + rh - 1) / rh;
-  return (unsigned)((tiles + kGemvWaves - 1) / kGemvWaves);
-}
-
-unsigned head_blocks(int64_t vocab, int K) {
-  const unsigned b = gemv_blocks(vocab, false), most = head_max_blocks(K);
-  return b > most ? most : b;
+  const unsigned b = (unsigned)((tiles + kGemvWaves - 1) / kGemvWaves);
+  return capped && b > kHeadMaxBlocks ? kHeadMaxBlocks : b;
 }
 
 template <int EPI, bool NORM, int XSRC = kXRow>
 int launch_fused(const FusedGemv& a, hipStream_t st) {
   const bool pairs = EPI == kEpiSwiGLU;
   const int rh = features_per_wave(a.N, pairs);
-  const unsigned blocks = EPI == kEpiArgmax ? head_blocks(a.N, a.K) : gemv_blocks(a.N, pairs);
+  const unsigned blocks = gemv_blocks(a.N, pairs, EPI == kEpiArgmax);
   const int nch = chunks_for(a.K);
   if constexpr (EPI == kEpiSwiGLU) {
     return launch_r<EPI, NORM, XSRC, 2>(a, nch, blocks, st);
@@ -927,6 +921,8 @@ int launch_fused(const FusedGemv& a, hipStream_t st) {
     return launch_r<EPI, NORM, XSRC, 1>(a, nch, blocks, st);
   }
 }
+
+unsigned head_blocks(int vocab) { return gemv_blocks(vocab, false, true); }
 
 struct StepLayout {
   size_t ml, acc, part_v, part_i, total;
@@ -938,7 +934,7 @@ StepLayout step_layout(const egpt_qwen3_step* s) {
   const size_t rows = (size_t)s->heads * (size_t)s->nsplit;
   L.ml = up(rows * sizeof(float));
   L.acc = up(rows * (size_t)s->head_dim * sizeof(float));
-  const size_t hb = head_blocks(s->vocab, s->hidden);
+  const size_t hb = head_blocks(s->vocab);
   L.part_v = up(hb * sizeof(float));
   L.part_i = up(hb * sizeof(int));
   L.total = 2 * L.ml + L.acc + L.part_v + L.part_i;
@@ -1178,7 +1174,7 @@ int gemv_few_rows(const void* x, int64_t ldx, const int8_t* w, int64_t ldw, cons
   a.y = (uint16_t*)y;
   a.y_ld = ldy;
   const int r = features_per_wave(N, false);  // the single-row kernel's tiles
-  const unsigned blocks = gemv_blocks(N, false);
+  const unsigned blocks = gemv_blocks(N, false, false);
   constexpr int W = kGemvWaves;
   const int nch = chunks_for(K);
 #define EGPT_ROWS(MM, RR, C) hipLaunchKernelGGL((gemv_rows_kernel<MM, RR, C, W>), dim3(blocks), dim3(W * kWave), 0, st, a)
@@ -1214,7 +1210,7 @@ using namespace egpt;
 
 extern "C" int egpt_int8_gemv_fused_parts(const egpt_gemv_fused* g, int* parts) {
   if (!g || !parts || g->N < 1) return EGPT_ERR_INVALID;
-  *parts = g->epilogue == EGPT_EPI_ARGMAX ? (int)head_blocks(g->N, g->K) : 0;
+  *parts = g->epilogue == EGPT_EPI_ARGMAX ? (int)gemv_blocks(g->N, false, true) : 0;
   return EGPT_OK;
 }
 
@@ -1318,7 +1314,7 @@ extern "C" int egpt_qwen3_decode_step(const egpt_qwen3_step* s, hipStream_t stre
   // head: final norm + lm_head + per-block maxima, then the greedy pick
   head_gemv(s, g);
   if ((st = run_fused(g[0], stream)) != EGPT_OK) return st;
-  const ArgmaxFinal f{g[0].part_v, g[0].part_i, (int)head_blocks(s->vocab, s->hidden), s->token, s->position, s->token_ring,
+  const ArgmaxFinal f{g[0].part_v, g[0].part_i, (int)head_blocks(s->vocab), s->token, s->position, s->token_ring,
                       s->token_ring ? s->token_ring_slots : 1};
   hipLaunchKernelGGL(argmax_final_kernel, dim3(1), dim3(kFThreads), 0, stream, f);
   return EGPT_LAUNCH_STATUS();

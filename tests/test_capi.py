@@ -126,3 +126,17 @@ def test_gemm_split_workspace_policy():
                               ((160, 4096, 2048), 0), ((256, 2048, 6144), 2), ((257, 2048, 2048), 0)):
         assert lib.egpt_int8_gemm_workspace(m, n, k, ctypes.byref(size)) == 0
         assert size.value == splits * m * n * 4, (m, n, k, size.value)
+
+
+@pytest.mark.parametrize('n', [512, 32000, 151936])
+def test_argmax_parts_follow_the_features_alone(n):
+    """The entries of an argmax GEMV's part_v / part_i: a caller may ask before it fills in K, and every K writes that
+    many."""
+    lib, g, parts = _lib.lib(), _lib.GemvFused(), ctypes.c_int()
+    g.epilogue, g.N = _lib.EPI_ARGMAX, n
+    seen = set()
+    for k in (0, 2048, 2064, 4096, 12288):
+        g.K = k
+        assert lib.egpt_int8_gemv_fused_parts(ctypes.byref(g), ctypes.byref(parts)) == 0
+        seen.add(parts.value)
+    assert len(seen) == 1 and 1 <= parts.value <= 1024
