@@ -83,7 +83,8 @@ __global__ __launch_bounds__(kThreads) void prompt_start_kernel(const int64_t* _
   }
 }
 
-// Byte offsets into the workspace.
+// Byte offsets into the workspace. qkv, qrot, attn and the decode attention's partials live from the QKV product to the
+// o product, gu and act from the gate/up product to the down product: the two groups share their memory.
 struct Layout {
   size_t positions, x, h, qkv, qrot, attn, o, gu, act, split, split_bytes, attn_ws, attn_ws_bytes, arg, arg_bytes, total;
   int attn_splits;
@@ -102,12 +103,7 @@ bool prompt_layout(const egpt_qwen3_step* s, int rows, Layout* out) {
   l.positions = take(r * sizeof(int64_t));
   l.x = take(r * s->hidden * 2);
   l.h = take(r * s->hidden * 2);
-  l.qkv = take(r * nqkv * 2);
-  l.qrot = take(r * nq * 2);
-  l.attn = take(r * nq * 2);
   l.o = take(r * s->hidden * 2);
-  l.gu = take(r * 2 * (size_t)s->inter * 2);
-  l.act = take(r * s->inter * 2);
   const int shape[4][2] = {{nqkv, s->hidden}, {s->hidden, nq}, {2 * s->inter, s->hidden}, {s->hidden, s->inter}};
   if (rows > EGPT_MAX_DECODE_ROWS)
     for (const auto& nk : shape) {
@@ -120,9 +116,17 @@ bool prompt_layout(const egpt_qwen3_step* s, int rows, Layout* out) {
   if (egpt_decode_attn_workspace(rows, s->heads, s->kv_heads, s->cap, D, l.attn_splits, &l.attn_ws_bytes) != EGPT_OK ||
       egpt_argmax_workspace(s->vocab, &l.arg_bytes) != EGPT_OK)
     return false;
-  l.attn_ws = take(l.attn_ws_bytes);
   l.arg = take(l.arg_bytes);
+  const size_t shared = at;
+  l.qkv = take(r * nqkv * 2);
+  l.qrot = take(r * nq * 2);
+  l.attn = take(r * nq * 2);
+  l.attn_ws = take(l.attn_ws_bytes);
   l.total = at;
+  at = shared;
+  l.gu = take(r * 2 * (size_t)s->inter * 2);
+  l.act = take(r * s->inter * 2);
+  if (at > l.total) l.total = at;
   *out = l;
   return true;
 }

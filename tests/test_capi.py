@@ -140,3 +140,29 @@ def test_argmax_parts_follow_the_features_alone(n):
         assert lib.egpt_int8_gemv_fused_parts(ctypes.byref(g), ctypes.byref(parts)) == 0
         seen.add(parts.value)
     assert len(seen) == 1 and 1 <= parts.value <= 1024
+
+
+@pytest.mark.parametrize('hidden,inter,heads,kv_heads,d,vocab,cap', [
+    (2048, 6144, 16, 8, 128, 151936, 8704), (4096, 12288, 32, 8, 128, 151936, 8704), (128, 256, 4, 2, 32, 512, 8704)])
+def test_prompt_workspace_is_no_larger_than_the_pass_tensors(hidden, inter, heads, kv_heads, d, vocab, cap):
+    """egpt_qwen3_prefill_workspace against one tensor per activation of the pass (x, h, qkv, q, attn, o, gate/up, act,
+    down), the positions, the largest split-K workspace and the argmax's, for prompts that run the prompt attention; below
+    its 64 rows the decode attention's partials come on top."""
+    lib, step, size = _lib.lib(), _lib.Qwen3Step(), ctypes.c_size_t()
+    step.layers, step.hidden, step.inter, step.heads, step.kv_heads = 2, hidden, inter, heads, kv_heads
+    step.head_dim, step.vocab, step.cap, step.eps = d, vocab, cap, 1e-6
+    step.nsplit = lib.egpt_qwen3_step_default_splits(heads, kv_heads, d, cap)
+    nq, nqkv = heads * d, (heads + 2 * kv_heads) * d
+    for rows in (1, 2, 16, 17, 64, 65, 100, 128, 300, 1000, 6001, 8192):
+        split = 0
+        for n, k in ((nqkv, hidden), (hidden, nq), (2 * inter, hidden), (hidden, inter)):
+            assert lib.egpt_int8_gemm_workspace(rows, n, k, ctypes.byref(size)) == 0
+            split = max(split, size.value if rows > 16 else 0)
+        assert lib.egpt_argmax_workspace(vocab, ctypes.byref(size)) == 0
+        most = 8 * rows + 2 * rows * (4 * hidden + nqkv + 2 * nq + 3 * inter) + split + size.value + 16 * 256
+        if rows < 65:
+            ns = step.nsplit if rows == 1 else lib.egpt_decode_attn_default_splits(rows, kv_heads, cap)
+            assert lib.egpt_decode_attn_workspace(rows, heads, kv_heads, cap, d, ns, ctypes.byref(size)) == 0
+            most += size.value
+        assert lib.egpt_qwen3_prefill_workspace(ctypes.byref(step), rows, ctypes.byref(size)) == 0
+        assert size.value <= most, (rows, size.value, most)
