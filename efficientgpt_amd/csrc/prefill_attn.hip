@@ -52,8 +52,17 @@ constexpr int kPfThreads = kPfWaves * 64;
 constexpr float kPfLog2e = 1.4426950408889634f;
 constexpr float kPfLazy = 8.f;  // exponent by which a score may pass the softmax's reference maximum (p < 2^8)
 
-// Blocks up to which a prompt takes the two-group form: its blocks, twice as many, still fit the 256 CUs in one round.
+// Blocks up to which a prompt may take the two-group form: its blocks, twice as many, still fit the 256 CUs in one round.
 constexpr int kPfSmallGrid = 128;
+
+// Whether such a prompt takes it. Sharing four tiles or more always gains. With two or three the pair staged first and the
+// merge cost about what the shorter chain saves, so only where the rows also fill more blocks of half the size (bt2
+// positions), or the rows of K and V are short (D 32). Measured on the MI355X, us, one group / two, 16 / 8 heads, D 128
+// (bt2 64): one tile, 64 rows 7.0 / 8.6; three, 65 rows over 127 slots 10.2 / 10.5, 64 over 127 10.1 / 10.5, 100 over 63
+// 1.26x; 32 / 8 heads (bt2 32), 65 over 127 1.19x; D 32, 4 / 2 heads, 33 to 128 rows 1.12-1.29x.
+constexpr bool two_groups(int tiles, int rows, int bt2, int D) {
+  return tiles >= 4 || (tiles >= 2 && (D == 32 || rows >= bt2 + 32));
+}
 
 struct PrefillArgs {
   const uint16_t* q;
@@ -423,7 +432,8 @@ extern "C" int egpt_prefill_attn(const void* q, int64_t q_ld, const void* k, con
     a.ntiles = (rows + a.bt - 1) / a.bt;
     return (int64_t)Hkv * (group / a.hb) * a.ntiles;
   };
-  const int kvg = blocks(1) <= kPfSmallGrid ? 2 : 1;
+  const int tiles = (pos0 + rows + kPfSlots - 1) / kPfSlots;
+  const int kvg = blocks(1) <= kPfSmallGrid && two_groups(tiles, rows, 32 * kPfWaves / 2 / a.hb, D) ? 2 : 1;
   blocks(kvg);
   const dim3 grid((unsigned)(Hkv * (group / a.hb)), (unsigned)a.ntiles);
 #define EGPT_PF(DD)                                                                                        \

@@ -89,8 +89,8 @@ def test_prefill_attention_small_head_dims_long_prompt(d):
 @pytest.mark.parametrize('hq,hkv', [(8, 2), (4, 2), (3, 3)])
 @pytest.mark.parametrize('rows,pos0', [(33, 0), (64, 0), (65, 0), (2, 126), (40, 88), (128, 64), (129, 191), (31, 257)])
 def test_prefill_attention_two_tile_groups(d, hq, hkv, rows, pos0):
-    """Small grids, whose wavefronts take the even and the odd tiles: one tile (the second group's state stays empty),
-    odd and even tile counts, a last tile of one slot, first rows that see no odd tile; against the oracle."""
+    """Small grids, on both sides of the rule by which their wavefronts take the even and the odd tiles: odd and even tile
+    counts, a last tile of one slot, first rows that see no odd tile; against the oracle."""
     q, k, v, _ = _case(rows, hq, hkv, pos0 + rows + 7, pos0, seed=rows + pos0 + d, D=d)
     _check(q, k, v, hq, hkv, pos0)
 
@@ -105,6 +105,19 @@ def test_prefill_attention_large_and_small_grids_agree(d, hq, hkv, rows, pos0):
     step = 517
     parts = torch.cat([_run(q[lo:lo + step], k, v, hq, hkv, pos0 + lo) for lo in range(0, rows, step)]).float()
     assert float((whole - parts).abs().max()) <= 2 ** -7 * float(v.abs().max()) + 2e-4
+
+
+@pytest.mark.parametrize('d,group,rows,pos0', [(128, 2, 64, 127), (128, 2, 65, 96), (128, 1, 128, 63), (64, 2, 64, 63),
+                                               (64, 4, 33, 127), (128, 2, 95, 30), (64, 1, 159, 30), (32, 2, 64, 0)])
+def test_prefill_attention_few_tiles_few_rows_keep_one_group(d, group, rows, pos0):
+    """Two or three tiles whose rows do not fill more of the smaller blocks (and a single tile) stay with one group of
+    wavefronts: the same bits as the same heads among so many that the grid is large (a head's arithmetic does not depend
+    on the other heads)."""
+    few, many = 2, 140
+    q, k, v, _ = _case(rows, many * group, many, pos0 + rows + 3, pos0, seed=rows + pos0, D=d)
+    large = _run(q, k, v, many * group, many, pos0)
+    small = _run(q[:, :few * group * d].contiguous(), k[:few], v[:few], few * group, few, pos0)
+    assert torch.equal(small, large[:, :few * group * d])
 
 
 def test_prefill_attention_qwen3_8b_heads_long_prompt():
