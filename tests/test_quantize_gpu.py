@@ -94,7 +94,8 @@ def test_ties_zero_rows_fp16_and_strides():
 
 
 @pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
-@pytest.mark.parametrize('k', [1, 3, 7, 8, 65, 511, 513, 1030, 2049, 4095, 4097, 9001, 16383, 16385, 33000])
+@pytest.mark.parametrize('k', [1, 3, 7, 8, 64, 65, 128, 129, 192, 193, 511, 513, 1030, 2049, 4095, 4097, 9001, 16383,
+                               16385, 33000])
 def test_row_lengths(dtype, k):
     """Row lengths at the edges of every form (shorter than a 16-byte chunk, each register count, one wavefront or a
     block per row, rows read twice), rows off 16-byte alignment, and the rows the multiplying form leaves to the
@@ -111,13 +112,22 @@ def test_row_lengths(dtype, k):
         # 127 (2 - 2^-23) rounds to a multiple whose 127th is 2 - 2^-23 again: a step of 24 ones
         w[6, 0] = 127 * (2 - 2.0 ** -23)
         w[6, 1:] = w[6, 1:].clamp(-200, 200)
-    w = w.contiguous() if k % 2 else w
-    finite = torch.cat([w, w])[:13].cuda()
+
+    def on_device(t):  # even k: rows inside a wider device matrix, off 16-byte alignment
+        if k % 2:
+            return t.contiguous().cuda()
+        wide = torch.full((13, k + 3), float('nan'), dtype=dtype, device='cuda')
+        wide[:, 1:k + 1] = t.cuda()
+        d = wide[:, 1:k + 1]
+        assert d.stride(0) == k + 3 and d.data_ptr() % 16 != 0
+        return d
+
+    finite = on_device(w)
     q, s = quantize_weight(finite)
     assert_same_as_oracle(finite, q, s)
     w[1, k // 2] = float('inf')
     w[2, k - 1] = float('nan')
-    d = w.cuda()
+    d = on_device(w)
     q, s = quantize_weight(d)
     keep = [r for r in range(13) if r not in (1, 2)]
     assert_same_as_oracle(d[keep], q[keep], s[keep])
@@ -127,6 +137,25 @@ def test_row_lengths(dtype, k):
     want = torch.zeros(k, dtype=torch.int8)
     want[k // 2] = -127
     assert torch.equal(q[1].cpu(), want) and bool((q[2] == -127).all())
+
+
+@pytest.mark.parametrize('dtype', [torch.bfloat16, torch.float16, torch.float32])
+@pytest.mark.parametrize('k', [1, 7, 100, 193, 511, 513, 1025, 2049, 4097, 9001, 16385, 33001, 140001])
+def test_output_rows_wider_than_k(dtype, k):
+    """egpt_quantize_rows into rows of a wider code matrix at an odd address: the codes and steps of the compact call, and
+    the bytes around every row as they were (a row's last chunks are moved back to end at K)."""
+    from efficientgpt_amd import _lib
+    from efficientgpt_amd.int8_linear import _QUANT_DTYPES, quantize_weight
+    n = 9
+    w = (torch.randn(n, k, generator=torch.Generator().manual_seed(k)) * 0.02).to(dtype).cuda()
+    want, steps = quantize_weight(w)
+    wide = torch.full((n, k + 24), 85, dtype=torch.int8, device='cuda')
+    s = torch.full((n + 2,), 7.0, device='cuda')
+    assert _lib.lib().egpt_quantize_rows(_QUANT_DTYPES[dtype], w.data_ptr(), k, n, k, wide.data_ptr() + 11, k + 24,
+                                         s.data_ptr() + 4, _lib.stream_ptr()) == 0
+    assert torch.equal(wide[:, 11:k + 11], want) and torch.equal(s[1:-1], steps)
+    assert bool((wide[:, :11] == 85).all()) and bool((wide[:, k + 11:] == 85).all())
+    assert float(s[0]) == 7 and float(s[-1]) == 7
 
 
 def test_quantize_model_on_gpu_matches_oracle_codes():
