@@ -8,6 +8,8 @@
 // (__fdiv_rn, or the multiplications of code_mul that give the same bits), so
 // the codes and steps are the bits of the formula evaluated on the CPU, whatever
 // the order of the max.
+#include <algorithm>
+
 #include "common.h"
 
 namespace egpt {
@@ -210,11 +212,18 @@ void launch_short(const T* w, int64_t ldw, int N, int K, int8_t* q, int64_t ldq,
                      ldw, N, K, q, ldq, s);
 }
 
+// A launch holds fewer than 2^32 threads: with a block per row, 2^23 rows take half of that.
+constexpr int kLaunchRows = 1 << 23;
+static_assert((uint64_t)kLaunchRows * kQuantWaves * kWave < (1ull << 32), "");
+
 template <typename T, int NC, int W>
 void launch_rows(const T* w, int64_t ldw, int N, int K, int8_t* q, int64_t ldq, float* s, hipStream_t st) {
   constexpr int kRows = kQuantWaves / W;
-  hipLaunchKernelGGL((quantize_rows_kernel<T, NC, W>), dim3((unsigned)(((int64_t)N + kRows - 1) / kRows)),
-                     dim3(kQuantWaves * kWave), 0, st, w, ldw, N, K, q, ldq, s);
+  for (int64_t n0 = 0; n0 < N; n0 += kLaunchRows) {
+    const int rows = (int)std::min<int64_t>(N - n0, kLaunchRows);
+    hipLaunchKernelGGL((quantize_rows_kernel<T, NC, W>), dim3((unsigned)((rows + kRows - 1) / kRows)),
+                       dim3(kQuantWaves * kWave), 0, st, w + n0 * ldw, ldw, rows, K, q + n0 * ldq, ldq, s + n0);
+  }
 }
 
 // Element by element up to 3 a lane, then one wavefront per row up to 8 chunks a lane (32 registers of row), then a block
