@@ -158,6 +158,16 @@ def test_output_rows_wider_than_k(dtype, k):
     assert float(s[0]) == 7 and float(s[-1]) == 7
 
 
+def test_rows_past_one_launch():
+    """2^23 rows go in one launch; the rows on both sides of that and the last ones, against the oracle."""
+    from efficientgpt_amd.int8_linear import quantize_weight
+    n, k = (1 << 23) + 7, 200
+    w = torch.empty(n, k, dtype=torch.bfloat16, device='cuda').normal_(generator=torch.Generator('cuda').manual_seed(1))
+    q, s = quantize_weight(w)
+    for lo, hi in ((0, 5), ((1 << 23) - 5, n)):
+        assert_same_as_oracle(w[lo:hi], q[lo:hi], s[lo:hi])
+
+
 def test_quantize_model_on_gpu_matches_oracle_codes():
     transformers = pytest.importorskip('transformers')
     from efficientgpt_amd.int8_linear import Int8Linear, quantize_model
