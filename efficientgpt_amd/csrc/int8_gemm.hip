@@ -9,10 +9,10 @@
 // GEMM; here the weights are converted on the chip, so they cross HBM once, as int8.
 //
 // Design:
-//   * Every tile runs v_mfma_f32_16x16x32_bf16 with its operands loaded straight into LDS, the weights as int8:
+//   * Aligned shapes run v_mfma_f32_16x16x32_bf16 tiles with their operands loaded straight into LDS, the weights as int8:
 //     128 x 128 to 256 x 256 for large products (int8_gemm_dma_kernel: eight wavefronts whose two halves take turns
-//     at the matrix cores), 32 x 64 to 128 x 64 for the others (int8_gemm_ring_kernel: more and shorter blocks).
-//     All sum an output in the same order, so its bits do not depend on the tile.
+//     at the matrix cores), 32 x 64 to 128 x 128 for the others (int8_gemm_ring_kernel: more and shorter blocks).
+//     All of these sum an output in the same order, so its bits do not depend on the tile.
 //   * int8 -> bf16 is exact: every value in [-127, 127] is a bf16.
 //   * Rows past M or N read a valid row and are never stored.
 //   * Split-K (short M, long K: too few output tiles to give every CU a block):
@@ -346,7 +346,9 @@ __global__ __launch_bounds__(kDmaWaves * kWave, 1) void int8_gemm_dma_kernel(con
 // 128 x 64 tiles staged through registers, on the MI355X with the weights out of cache (us): 20 x 4096 -> 24576 SwiGLU
 // 36 -> 26, 77 x 2048 -> 12288 SwiGLU 20.4 -> 14.2, 200 x 4096 -> 6144 31.6 -> 26.7, 300 x 12288 -> 4096 97 -> 64, 300 x
 // 4096 -> 6144 42.5 -> 30, 600 x 2048 -> 2048 18.8 -> 13.1, 600 x 6144 -> 2048 51 -> 32.5; split slices 20 x 12288 ->
-// 4096 18.5 -> 16.5, at 64-128 rows within 3%.
+// 4096 18.5 -> 16.5. As 128 x 128 it also replaces int8_gemm_dma_kernel's where the blocks are one round: 1000 x 12288 ->
+// 4096 126 -> 111 us, 2048 x 6144 -> 2048 66 -> 58, 512 x 2048 -> 6144 24.4 -> 21.6 (a block is all a CU holds; that
+// kernel's fits twice and stays for two rounds).
 constexpr int kRingBK = 128;
 
 // LDS positions of a stage's 16-byte chunks: chunk c of x row r (16 a row) sits at c ^ (r & 15), chunk c of the weight
@@ -573,9 +575,14 @@ int launch_ring(GemmArgs a, hipStream_t st) {
   return EGPT_LAUNCH_STATUS();
 }
 
-// The split slices' fp32 tiles into a.part (a.splits > 1); no reduce.
+// The split slices' fp32 tiles into a.part (a.splits > 1); no reduce. Tiles of 32 rows for up to 32 rows and where the
+// 64-row ones are more than one round of 256 blocks (three of the smaller fit on a CU): 64 x 2048 -> 6144 (384 blocks) 12.7
+// -> 12.0 us, 192 x 2048 -> 2048 9.5 -> 8.9, 128 x 2048 -> 6144 16.1 -> 15.6; at 256 blocks 64 x 4096 -> 4096 12.0 ->
+// 12.2; 33 x 4096 -> 6144 14.2 -> 14.8.
 int launch_split_partials(const GemmArgs& a, hipStream_t st) {
-  if (a.M <= 32) return launch_ring<32, 64, 1, 4, 3, true, false>(a, st);
+  const int64_t blocks = ((int64_t)a.M + 63) / 64 * (((int64_t)a.N + 63) / 64) * a.splits;
+  const int last = (a.M - 1) % 64 + 1;  // rows of the last 64; a second 32 of a few rows is not worth its blocks
+  if (a.M <= 32 || (blocks > 256 && (last <= 32 || last >= 40))) return launch_ring<32, 64, 1, 4, 3, true, false>(a, st);
   return launch_ring<64, 64, 2, 4, 3, true, false>(a, st);
 }
 
@@ -624,8 +631,9 @@ constexpr GemmTile ring_tile(float round, float pair = 0.f) {
 constexpr GemmTile kGemmTiles[] = {
     dma_tile<8, 4>(95.0f), dma_tile<6, 4>(79.5f), dma_tile<8, 3>(79.5f), dma_tile<6, 3>(65.3f), dma_tile<4, 4>(61.7f),
     dma_tile<8, 2>(59.5f), dma_tile<4, 3>(53.8f), dma_tile<6, 2>(50.0f), dma_tile<4, 2>(39.7f, 64.0f),
-    ring_tile<64, 128, 2, 4, 4>(26.5f), ring_tile<128, 64, 2, 4, 3>(23.6f), ring_tile<96, 64, 2, 4, 3>(21.3f),
-    ring_tile<64, 64, 2, 4, 3>(17.3f, 27.0f), ring_tile<32, 64, 1, 4, 3>(14.0f, 24.0f)};
+    ring_tile<128, 128, 2, 4, 3>(36.0f), ring_tile<64, 128, 2, 4, 4>(26.5f), ring_tile<128, 64, 2, 4, 3>(23.6f),
+    ring_tile<96, 64, 2, 4, 3>(21.3f), ring_tile<64, 64, 2, 4, 3>(17.3f, 27.0f),
+    ring_tile<32, 64, 1, 4, 3>(14.0f, 24.0f)};
 
 float tile_cost(const GemmTile& t, int64_t M, int64_t N) {
   const int64_t tiles = ((M + t.bm - 1) / t.bm) * ((N + t.bn - 1) / t.bn);
@@ -635,11 +643,16 @@ float tile_cost(const GemmTile& t, int64_t M, int64_t N) {
 }
 
 // N counts a SwiGLU product's gate and up columns.
-int launch_best_tile(const GemmArgs& a, bool swiglu, hipStream_t st) {
+const GemmTile& best_tile(int64_t M, int64_t N, bool swiglu) {
   const GemmTile* best = nullptr;
   for (const GemmTile& t : kGemmTiles)
-    if ((t.swiglu || !swiglu) && (!best || tile_cost(t, a.M, a.N) < tile_cost(*best, a.M, a.N))) best = &t;
-  return swiglu ? best->launch_swiglu(a, st) : best->launch(a, st);
+    if ((t.swiglu || !swiglu) && (!best || tile_cost(t, M, N) < tile_cost(*best, M, N))) best = &t;
+  return *best;
+}
+
+int launch_best_tile(const GemmArgs& a, bool swiglu, hipStream_t st) {
+  const GemmTile& t = best_tile(a.M, a.N, swiglu);
+  return swiglu ? t.launch_swiglu(a, st) : t.launch(a, st);
 }
 
 // Any K, alignment and size: 64 x 64 of y per block, four wavefronts as 2 x 2. The tiles above need 16-byte aligned rows
