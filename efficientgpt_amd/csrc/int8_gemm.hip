@@ -612,6 +612,7 @@ struct GemmTile {
   int bm, bn;
   float round;  // 256 blocks
   float pair;   // 512 blocks, where two fit on a CU
+  bool ring;    // int8_gemm_ring_kernel, else int8_gemm_dma_kernel
   bool swiglu;  // has the SwiGLU form
   int (*launch)(GemmArgs, hipStream_t);
   int (*launch_swiglu)(GemmArgs, hipStream_t);
@@ -619,13 +620,13 @@ struct GemmTile {
 template <int TM, int TN>
 constexpr GemmTile dma_tile(float round, float pair = 0.f) {
   if constexpr (TN % 2 == 0)
-    return {32 * TM, 64 * TN, round, pair, true, launch_dma<TM, TN, false>, launch_dma<TM, TN, true>};
+    return {32 * TM, 64 * TN, round, pair, false, true, launch_dma<TM, TN, false>, launch_dma<TM, TN, true>};
   else
-    return {32 * TM, 64 * TN, round, pair, false, launch_dma<TM, TN, false>, nullptr};
+    return {32 * TM, 64 * TN, round, pair, false, false, launch_dma<TM, TN, false>, nullptr};
 }
 template <int BM, int BN, int WM, int WN, int STAGES>
 constexpr GemmTile ring_tile(float round, float pair = 0.f) {
-  return {BM, BN, round, pair, true, launch_ring<BM, BN, WM, WN, STAGES, false, false>,
+  return {BM, BN, round, pair, true, true, launch_ring<BM, BN, WM, WN, STAGES, false, false>,
           launch_ring<BM, BN, WM, WN, STAGES, false, true>};
 }
 constexpr GemmTile kGemmTiles[] = {
@@ -886,6 +887,15 @@ extern "C" int egpt_int8_gemm_workspace(int M, int N, int K, size_t* bytes) {
   int splits, kchunk;
   gemm_split(M, N, K, splits, kchunk);
   *bytes = splits > 1 ? (size_t)splits * (size_t)M * (size_t)N * sizeof(float) : 0;
+  return EGPT_OK;
+}
+
+extern "C" int egpt_int8_gemm_tile(int M, int N, int swiglu, int* rows, int* columns, int* ring) {
+  if (M < 1 || N < 1 || !rows || !columns || !ring) return EGPT_ERR_INVALID;
+  const GemmTile& t = best_tile(M, N, swiglu != 0);
+  *rows = t.bm;
+  *columns = t.bn;
+  *ring = t.ring;
   return EGPT_OK;
 }
 

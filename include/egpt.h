@@ -86,12 +86,15 @@ int egpt_quantize_rows(int dtype, const void *w, int64_t ldw, int N, int K, int8
  * without materialising the bf16 weights. x bf16 [M, K] (row stride ldx), w int8 [N, K]
  * (ldw), y bf16 [M, N] (ldy). The MFMA kernel takes K a multiple of 64, ldx % 8 == 0,
  * ldw % 16 == 0, 16-byte aligned x and w and operands under 2 GiB; any other shape runs
- * a kernel of 64 x 64 MFMA tiles with loads of any alignment, slower but
+ * 64 x 64 MFMA tiles with loads of any alignment (small ones a vector kernel), slower but
  * with the same contract.
  */
 int egpt_int8_gemm(const void *x, int64_t ldx, const int8_t *w, int64_t ldw, const float *scale,
                    void *y, int64_t ldy, int M, int N, int K, hipStream_t stream);
-/* The same product with a workspace, which lets short-M shapes (M <= 128 whose
+/* The tile that egpt_int8_gemm (swiglu 0) or egpt_int8_gemm_swiglu (1; N = 2 inter) runs for an aligned M x N
+ * product: rows and weight rows per block, and whether it is of the small tiles' kernel (*ring 1) or the large ones'. */
+int egpt_int8_gemm_tile(int M, int N, int swiglu, int *rows, int *columns, int *ring);
+/* The same product with a workspace, which lets short-M shapes (M <= 256 whose
  * 64 x 64 output tiles leave CUs idle) split K: each split's fp32 tile goes to the
  * workspace and a second launch adds the splits in order, then rounds as above.
  * egpt_int8_gemm_workspace gives the bytes the split needs for this shape (0: no

@@ -166,3 +166,18 @@ def test_prompt_workspace_is_no_larger_than_the_pass_tensors(hidden, inter, head
             most += size.value
         assert lib.egpt_qwen3_prefill_workspace(ctypes.byref(step), rows, ctypes.byref(size)) == 0
         assert size.value <= most, (rows, size.value, most)
+
+
+def test_every_gemm_tile_is_one_that_a_test_runs():
+    """The tiles that products of any size take (egpt_int8_gemm_tile) are those whose shapes the GPU tests name; they check
+    the names themselves, so a changed cost cannot leave a tile untested."""
+    import test_int8_linear_gpu as gpu
+    sizes = sorted({int(1.13 ** i) for i in range(1, 90)} | {9344, 890, 18440})
+    for swiglu, lists in ((False, (gpu.DMA_TILE_SHAPES, gpu.RING_TILE_SHAPES)),
+                          (True, (gpu.DMA_SWIGLU_SHAPES, gpu.RING_TILE_SHAPES))):
+        taken = {gpu.gemm_tile(m, 2 * n, swiglu) for m in sizes for n in sizes}
+        assert taken == {t[0] for shapes in lists for t in shapes}
+        for tile, m, _, n in lists[0]:
+            assert gpu.gemm_tile(m, 2 * n if swiglu else n, swiglu) == tile
+        for tile, m, _, n in lists[1]:
+            assert gpu.gemm_tile(m, n // 2 * 2 if swiglu else n, swiglu) == tile

@@ -116,7 +116,7 @@ def test_splitk_configs(m, k, n, config):
     check_against_oracle(y, x, q, s)
 
 
-def test_unaligned_and_strided_operands_take_the_generic_path():
+def test_unaligned_and_strided_operands():
     from efficientgpt_amd.int8_linear import int8_matmul
     x, q, s = make_case(2, 2051, 33, seed=4)
     big = torch.zeros(2, 2051 + 3, dtype=torch.bfloat16)
@@ -291,11 +291,25 @@ def test_prefill_gemm_kernel_matches_oracle(m, k, n):
     assert float((diff == 0).float().mean()) >= 0.9
 
 
-# 32 TM x 64 TN tiles of the LDS-direct kernel and shapes that take each: 1 to 4 K steps (the pipeline's prologue and
-# tail), ragged rows and features, an odd output pitch (stores off 16-byte alignment)
-DMA_TILE_SHAPES = [('4x2', 77, 192, 18441), ('6x2', 130, 64, 18440), ('4x3', 200, 128, 18443), ('4x4', 300, 256, 18440),
+def gemm_tile(m, n, swiglu):
+    """The name of the tile an aligned product takes: TM x TN of the large tiles (32 TM rows, 64 TN columns), rows x columns
+    of the small ones."""
+    import ctypes
+    from efficientgpt_amd import _lib
+    rows, columns, ring = ctypes.c_int(), ctypes.c_int(), ctypes.c_int()
+    assert _lib.lib().egpt_int8_gemm_tile(m, n, int(swiglu), rows, columns, ring) == 0
+    return f'{rows.value}x{columns.value}' if ring.value else f'{rows.value // 32}x{columns.value // 64}'
+
+
+# 32 TM x 64 TN tiles of the large tiles' kernel and shapes that take each: 1 to 4 and 11 to 17 K steps through three
+# stages (the pipeline's prologue, its cycle and its tail), ragged rows and features, an odd output pitch (stores off 16-byte
+# alignment)
+DMA_TILE_SHAPES = [('4x2', 9344, 192, 890), ('6x2', 130, 64, 18440), ('4x3', 200, 128, 18443), ('4x4', 300, 256, 18440),
                    ('8x2', 500, 192, 12300), ('6x4', 700, 192, 12300), ('8x4', 1000, 128, 12301),
-                   ('6x3', 1300, 192, 6150), ('8x3', 2500, 64, 14002)]
+                   ('6x3', 1300, 192, 6150), ('8x3', 2500, 64, 14002), ('4x2', 9300, 704, 890), ('6x2', 130, 768, 18440),
+                   ('4x3', 200, 832, 18443), ('4x4', 300, 704, 18440), ('8x2', 500, 1088, 12300),
+                   ('6x4', 700, 768, 12300), ('8x4', 1000, 704, 12301), ('6x3', 1300, 1088, 6150),
+                   ('8x3', 2500, 832, 14002)]
 
 
 @pytest.mark.parametrize('tile,m,k,n', DMA_TILE_SHAPES)
@@ -303,6 +317,7 @@ def test_prefill_gemm_lds_direct_tiles_match_oracle(tile, m, k, n):
     """Every tile of the LDS-direct GEMM against the oracle's prefill formula; rows and columns past the output stay
     untouched."""
     from efficientgpt_amd import _lib
+    assert gemm_tile(m, n, False) == tile
     x, q, s = make_case(m, k, n, seed=m + k + n)
     xd, qd, sd = x.cuda(), q.cuda(), s.cuda()
     y = torch.full((m + 1, n + 3), 7.0, device='cuda', dtype=torch.bfloat16)
@@ -313,12 +328,17 @@ def test_prefill_gemm_lds_direct_tiles_match_oracle(tile, m, k, n):
     assert bool((y[m] == 7).all()) and bool((y[:, n:] == 7).all())
 
 
-@pytest.mark.parametrize('tile,m,k,inter', [('4x2', 77, 192, 9221), ('6x2', 130, 64, 9220), ('8x2', 200, 128, 9223),
-                                            ('4x4', 300, 256, 9220), ('6x4', 1300, 192, 3075), ('8x4', 1000, 64, 6150)])
+DMA_SWIGLU_SHAPES = [('4x2', 9344, 192, 445), ('6x2', 130, 64, 9220), ('8x2', 200, 128, 9223), ('4x4', 300, 256, 9220),
+                     ('6x4', 1300, 192, 3075), ('8x4', 1000, 64, 6150), ('4x2', 9300, 704, 445), ('6x2', 130, 1088, 9220),
+                     ('8x4', 1000, 704, 6150)]
+
+
+@pytest.mark.parametrize('tile,m,k,inter', DMA_SWIGLU_SHAPES)
 def test_gemm_swiglu_lds_direct_tiles_match_the_two_calls(tile, m, k, inter):
     """The SwiGLU form of every LDS-direct tile it has, bit for bit against the product followed by egpt_silu_mul."""
     from efficientgpt_amd import _lib
     lib = _lib.lib()
+    assert gemm_tile(m, 2 * inter, True) == tile
     x, q, s = make_case(m, k, 2 * inter, seed=m + inter)
     xd, qd, sd = x.cuda(), q.cuda(), s.cuda()
     gu = torch.empty(m, 2 * inter, device='cuda', dtype=torch.bfloat16)
@@ -339,7 +359,8 @@ def test_gemm_swiglu_lds_direct_tiles_match_the_two_calls(tile, m, k, inter):
 RING_TILE_SHAPES = [('32x64', 20, 64, 77), ('32x64', 17, 192, 200), ('32x64', 100, 1088, 130), ('64x64', 256, 128, 4090),
                     ('64x64', 100, 2112, 8000), ('64x64', 190, 320, 5300), ('96x64', 77, 192, 12290),
                     ('96x64', 96, 576, 12290), ('128x64', 120, 320, 12290), ('128x64', 250, 448, 6150),
-                    ('64x128', 60, 64, 20001), ('64x128', 190, 704, 9000)]
+                    ('64x128', 60, 64, 20001), ('64x128', 190, 704, 9000), ('128x128', 77, 192, 18441),
+                    ('128x128', 77, 64, 18442), ('128x128', 1000, 2112, 4090), ('128x128', 500, 576, 6150)]
 
 
 @pytest.mark.parametrize('tile,m,k,n', RING_TILE_SHAPES)
@@ -348,6 +369,7 @@ def test_prefill_gemm_small_tiles_match_oracle(tile, m, k, n):
     with an even feature count egpt_int8_gemm_swiglu against the same product followed by egpt_silu_mul, bit for bit."""
     from efficientgpt_amd import _lib
     lib = _lib.lib()
+    assert gemm_tile(m, n, False) == tile
     x, q, s = make_case(m, k, n, seed=m + k + n)
     xd, qd, sd = x.cuda(), q.cuda(), s.cuda()
     y = torch.full((m, n + 3), -7.0, device='cuda', dtype=torch.bfloat16)
@@ -357,6 +379,7 @@ def test_prefill_gemm_small_tiles_match_oracle(tile, m, k, n):
     assert bool((y[:, n:] == -7).all())
     if n % 2 or k % 128 == 0:
         return
+    assert gemm_tile(m, n, True) == tile
     inter = n // 2
     gu = y[:, :n].contiguous()
     two, one = (torch.full((m, inter), -7.0, device='cuda', dtype=torch.bfloat16) for _ in range(2))
@@ -402,13 +425,13 @@ def test_prefill_gemm_split_k_matches_oracle(m, k, n):
     assert torch.equal(int8_linear(xd, qd, sd), y)
 
 
-GENERIC_SHAPES = [(40, 100, 70), (17, 2051, 33), (64, 96, 257)]
+UNALIGNED_SHAPES = [(40, 100, 70), (17, 2051, 33), (64, 96, 257)]
 
 
-@pytest.mark.parametrize('m,k,n', GENERIC_SHAPES)
-def test_prefill_generic_kernel_for_shapes_the_mfma_kernel_refuses(m, k, n):
-    """K not a multiple of 64, and x rows 6 bytes off 16-byte alignment: egpt_int8_gemm runs its generic
-    kernel (no library formula anywhere in the op) with the prefill formula's two roundings, against the oracle."""
+@pytest.mark.parametrize('m,k,n', UNALIGNED_SHAPES)
+def test_prefill_kernels_for_shapes_off_alignment(m, k, n):
+    """K not a multiple of 64, and x rows 6 bytes off 16-byte alignment: egpt_int8_gemm's kernels of any alignment
+    (no library formula anywhere in the op) with the prefill formula's two roundings, against the oracle."""
     from efficientgpt_amd import _lib
     from efficientgpt_amd.int8_linear import int8_linear
     x, q, s = make_case(m, k, n, seed=m + k + n)
