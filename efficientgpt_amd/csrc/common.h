@@ -92,7 +92,8 @@ __device__ __forceinline__ void gstore(T* p, T v) {
 
 __device__ __forceinline__ u32x4 ld16(const void* p) { return *(global_ptr<const u32x4>)p; }
 
-// 16 bytes from any address (the target takes unaligned vector accesses).
+// 16 bytes at any element of a 16-bit row, and from any address (the target takes unaligned vector accesses).
+typedef uint32_t u32x4_h __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x4_b __attribute__((ext_vector_type(4), aligned(1)));
 __device__ __forceinline__ u32x4 ld16_any(const void* p) { return *(global_ptr<const u32x4_b>)p; }
 

@@ -121,7 +121,6 @@ constexpr int kDmaStages = 3;
 __device__ __forceinline__ int dma_aswz(int r) { return ((r >> 1) & 1) | (((r >> 3) & 1) << 2); }
 __device__ __forceinline__ int dma_bswz(int t) { return ((t & 1) << 1) ^ (3 * ((t >> 1) & 1)); }
 
-typedef uint32_t u32x4_h __attribute__((ext_vector_type(4), aligned(2)));
 typedef uint32_t u32x2_h __attribute__((ext_vector_type(2), aligned(2)));
 typedef uint32_t u32_h __attribute__((aligned(2)));
 typedef float f32x4_w __attribute__((ext_vector_type(4), aligned(4)));
@@ -858,7 +857,12 @@ int launch_ragged(GemmArgs a, hipStream_t st) {
 // K slices for a short-M GEMM (at most 256 rows) whose 64 x 64 tiles leave CUs
 // idle: the fewest (a power of two, at most 16) that give every CU a block, each
 // slice a multiple of kBKSplit and at least 256 wide. 1 when the tiles already fill
-// the chip, or K is short or not a multiple of kBKSplit.
+// the chip, or K is short or not a multiple of kBKSplit. The rule was chosen on tiles
+// that are gone; with the present ones, us, split (slices and reduce) / one pass: where
+// K is long it gains, 128 x 12288 -> 4096 31.0 / 41.3, 128 x 6144 -> 2048 12.4 / 21.8,
+// 64 x 2048 -> 2048 6.7 / 8.9; where two slices do, 32 x 64 tiles would fill the chip
+// in one pass and it loses, 128 x 2048 -> 4096 11.3 / 9.1, 64 x 2048 -> 12288 16.2 /
+// 12.8, 200 x 2048 -> 2048 9.6 / 9.0.
 constexpr int kMinSliceSteps = 4;
 constexpr int kSplitTargetBlocks = 256;
 
@@ -867,9 +871,7 @@ void gemm_split(int64_t M, int64_t N, int64_t K, int& splits, int& kchunk) {
   splits = 1;
   kchunk = (int)K;
   if (M > 256 || K % kBKSplit) return;  // taller blocks take the larger tiles below
-  // Past 128 rows only grids that fill at most half the CUs split (measured on the
-  // MI355X: 200 x 2048 -> 2048, 128 tiles, 12.6 -> 10.1 us with 2 splits; 160 x 2048
-  // -> 4096, 192 tiles, 13.4 -> 16.2 us with 2)
+  // Past 128 rows only grids that fill at most half the CUs split.
   if (M > 128 && tiles > kSplitTargetBlocks / 2) return;
   while (tiles * splits < kSplitTargetBlocks && splits < kMaxSplits && K / (2 * splits) >= kMinSliceSteps * kBK) splits *= 2;
   if (splits == 1) return;

@@ -76,10 +76,9 @@ __device__ __forceinline__ bool step_multiplies(float step) {
 
 // 16 bytes of a weight row at any element alignment, and 4 or 8 codes at any byte alignment (the target takes
 // unaligned vector accesses; aligned rows lose nothing by the wider type).
-typedef uint32_t u32x4_el __attribute__((ext_vector_type(4), aligned(2)));
 template <typename T>
 __device__ __forceinline__ u32x4 ld16_el(const T* p) {
-  return __builtin_nontemporal_load((global_ptr<const u32x4_el>)p);
+  return __builtin_nontemporal_load((global_ptr<const u32x4_h>)p);
 }
 typedef uint32_t u32_any __attribute__((aligned(1)));
 typedef uint32_t u32x2_any __attribute__((ext_vector_type(2), aligned(1)));

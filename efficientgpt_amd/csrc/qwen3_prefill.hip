@@ -17,7 +17,6 @@ namespace egpt {
 namespace {
 
 constexpr int kThreads = 256;
-typedef uint32_t u32x4_h __attribute__((ext_vector_type(4), aligned(2)));
 
 // Row r of the prompt: x = table[token], h = RMSNorm(x) * w, positions[r] = pos0 + r; block 0 sets *position to the last
 // row's. The sums run in add_rmsnorm_kernel's order (V8: add_rmsnorm_v8_kernel's), so x and h have the bits of

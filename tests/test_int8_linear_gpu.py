@@ -389,6 +389,23 @@ def test_prefill_gemm_small_tiles_match_oracle(tile, m, k, n):
     assert torch.equal(one, two)
 
 
+@pytest.mark.parametrize('m,k,n', [(128, 2048, 4096), (128, 2048, 2048), (128, 2048, 12288), (128, 6144, 2048),
+                                   (77, 4096, 6144), (600, 4096, 4096), (1500, 4096, 24576), (1500, 12288, 4096),
+                                   (300, 4001, 1000), (40, 7001, 3000)])
+def test_prefill_gemm_is_exact_where_the_sums_are(m, k, n):
+    """Whole-number activations up to 4: every partial sum is a whole number below 2^24, exact in fp32 in any order, so the
+    outputs are the formula's bits whatever the tile, the split or the matrix instruction. Products of other values differ
+    between those by the order of their sums alone."""
+    from efficientgpt_amd.int8_linear import int8_linear
+    g = torch.Generator(device='cuda').manual_seed(m + n)
+    x = torch.randint(-4, 5, (m, k), generator=g, device='cuda').to(torch.bfloat16)
+    q = torch.randint(-127, 128, (n, k), generator=g, device='cuda', dtype=torch.int8)
+    s = torch.rand(n, generator=g, device='cuda') * 0.02 + 1e-3
+    total = x.double() @ q.t().double()
+    assert float(total.abs().max()) < 2 ** 24
+    assert torch.equal(int8_linear(x, q, s), (total.float().to(torch.bfloat16).float() * s).to(torch.bfloat16))
+
+
 SPLIT_SHAPES = [(128, 6144, 2048), (128, 2048, 4096), (33, 6144, 2048), (64, 2048, 2048), (100, 4096, 1000),
                 (17, 12288, 64), (200, 2048, 2048), (130, 2048, 2000), (256, 2048, 2048)]
 
