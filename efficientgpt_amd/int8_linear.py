@@ -99,10 +99,9 @@ def int8_gemm(x2, w, s, out=None, workspace=None):
     """Prefill rows: bf16(fp32(bf16(x2 @ w^T)) * s), the reference's formula for more than 16 rows
     (research/realmodel/int8_linear.py:96-97), on the MFMA kernel egpt_int8_gemm, which reads the int8 weights
     directly (no bf16 copy of them). Measured on the MI355X against the reference's dequantise-then-library-GEMM
-    formula at the Qwen3-1.7B and Qwen3-8B shapes: 1.2-2.9x faster at 128 rows, 1.1-1.4x at 1024-2048, and at
-    8192 rows 0.93-1.4x (faster on 14 of 16 shapes, the whole 8B layer 8% faster). Shapes the MFMA kernel does
-    not take (K not a multiple of 64, unaligned rows, operands of 2 GiB or more) run the library's ragged kernel,
-    the same formula on smaller tiles with loads of any alignment."""
+    formula at the Qwen3-1.7B and Qwen3-8B shapes, weights in cache: 3.3-7.2x its speed at 128 rows, 1.6-2.7x at
+    1024-2048, 1.3-2.0x at 8192. Shapes those tiles do not take (K not a multiple of 64, unaligned rows, operands of
+    2 GiB or more) run the library's kernels of any alignment, the same formula on smaller tiles."""
     m, k = x2.shape
     n = w.shape[0]
     if x2.stride(1) != 1:
