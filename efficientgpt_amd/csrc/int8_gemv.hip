@@ -133,10 +133,10 @@ __global__ __launch_bounds__(kGemvThreads) void gemv_i8_rows(
 
 // Any alignment, strides and K of at least 16 columns per split: one wavefront per output row, 16 columns a lane with
 // loads of any alignment, each weight converted once for up to four activation rows (grid z; 16 rows in one block took
-// 256 registers and left two wavefronts a SIMD: 16 x 520 -> 8192 59 us, in groups of four 21). The codes are converted signed: the
-// biased form above would make x * (w + 128) and 128 * x of an infinite or very large x cancel into NaN, and sums with a
-// mean several times less exact; these kernels keep the plain sum of x * w. The lane that a slice ends in moves its
-// chunk back to end there, with zeros for the activations that the lane before it has.
+// 256 registers and left two wavefronts a SIMD: 16 x 520 -> 8192 59 us, in groups of four 21). The codes are converted
+// signed: the biased form above would make x * (w + 128) and 128 * x of an infinite or very large x cancel into NaN, and
+// sums with a mean several times less exact; these kernels keep the plain sum of x * w. The lane that a slice ends in
+// moves its chunk back to end there, with zeros for the activations that the lane before it has.
 template <int M, int EPI>
 __global__ __launch_bounds__(kGemvThreads) void gemv_i8_ragged(
     const uint16_t* __restrict__ x, int64_t ldx, const int8_t* __restrict__ w, int64_t ldw,

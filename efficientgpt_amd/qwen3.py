@@ -527,14 +527,15 @@ class Qwen3Int8Engine:
             raise ValueError('prompt exceeds the cache capacity')
         lib = _lib.lib()
         # The descriptor holds the addresses the engine was built with. Where a tensor has been replaced since (a layer's
-        # weight, the cache), the calls below take the tensors themselves, with the strides they have.
-        if self.fold_norms and self._tensor_addresses() == self._step_tensors:
+        # weight, the cache), the calls below take the tensors themselves, with the strides they have; and positions below
+        # zero, which each of their kernels clamps.
+        if self.fold_norms and pos0 >= 0 and self._tensor_addresses() == self._step_tensors:
             need = ctypes.c_size_t()
             _lib.check('egpt_qwen3_prefill_workspace', lib.egpt_qwen3_prefill_workspace(ctypes.byref(self._step_c), t,
                                                                                         ctypes.byref(need)))
             ws = torch.empty(need.value, device=dev, dtype=torch.uint8)
             _lib.check('egpt_qwen3_prefill', lib.egpt_qwen3_prefill(
-                ctypes.byref(self._step_c), ids.data_ptr(), t, pos0, int(use_prompt_kernel(t, pos0)), ws.data_ptr(),
+                ctypes.byref(self._step_c), ids.data_ptr(), t, int(pos0), int(use_prompt_kernel(t, pos0)), ws.data_ptr(),
                 need.value, self._stream()))
             return self.logits[0]
         positions = torch.arange(pos0, pos0 + t, device=dev, dtype=torch.long)

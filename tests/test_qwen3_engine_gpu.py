@@ -222,6 +222,20 @@ def test_prefill_reads_the_tensors_the_engine_holds(plen):
     assert torch.equal(eng.prefill(prompt), changed)
 
 
+def test_prefill_takes_every_kind_of_position():
+    """A position given as a float, a numpy integer or a tensor is the same as the int; one below zero is accepted (every
+    kernel clamps a row's position to the cache) and leaves position = pos0 + len."""
+    eng, _ = build(SMALL, seed=5, std=0.15, cap=128)
+    prompt = torch.randint(0, SMALL.vocab, (20,), generator=torch.Generator().manual_seed(2))
+    want = eng.prefill(prompt, 3).clone()
+    for pos0 in (3.0, np.int64(3), torch.tensor(3), torch.tensor(3, device='cuda')):
+        eng.reset()
+        assert torch.equal(eng.prefill(prompt, pos0), want) and int(eng.position) == 23
+    eng.reset()
+    eng.prefill(prompt, -1)
+    assert int(eng.position) == 19
+
+
 @pytest.mark.parametrize('shape', [SMALL, SMALL8])
 @pytest.mark.parametrize('plen', [40, 128, 4096])
 def test_prefill_folded_norms_equal_separate_calls(shape, plen):
